@@ -384,272 +384,6 @@ __global__ __launch_bounds__(AP_NT) void k_attn_pv(const float* __restrict__ S, 
 }
 
 
-// ---------------------------------------------------------------------------
-// k_attn_pvt: softmax and P.V for prefill, register-tiled.  Workgroup (kv
-// head, tile of qt = 32 / G queries): R = 32 score rows, all HD dims.  The
-// rows come into LDS by direct-to-LDS loads and go through the same softmax
-// as k_attn_pv (max; exp polynomial on the 8-aligned part, expf on the tail;
-// the reference's eight sum lanes, eng_hsum256 and the tail in order;
-// 1 / (sum + 1e-12)), and are normalised in place once (p = e * inv, the
-// reference's multiply).  Thread (ri, di) then keeps the 4 x 4 outputs of
-// rows ri + 8k (k < 4) and dims 4di .. 4di + 3 in registers and runs each
-// output's chain a = fma(p[t], v[t], a) over the keys in order: per 4 keys
-// one float4 of p per row from LDS and one float4 of V per key, 64 FMAs.  V
-// comes from L2 straight into registers, PVT_KV keys a batch with the next
-// batch in flight: the eight lanes of a wave that share a row group hold
-// eight consecutive float4 of the key's row, one 128-byte read per wave.
-// Keys at or past a row's kv_len (only the tile's last few keys: its rows end
-// at consecutive positions) leave that row's chains untouched.  G even (no
-// single trailing head), HD in {64, 128, 256}.
-// ---------------------------------------------------------------------------
-#define PVT_R 32  // score rows per workgroup (a multiple of 8 PVT_RT)
-#define PVT_RT 4  // rows per thread in P.V (workgroup of 8 HD / PVT_RT threads)
-#define PVT_KV 8  // keys per register batch of V
-
-// p of keys t .. t + 3 for the thread's RT rows (t clamped into the row so a
-// read ahead of the last keys stays inside it; such values are not used)
-template <int RT>
-DEV void pvt_readp(const float* pr, int ldp, int rs, int t, float4 (&p4)[RT]) {
-    t = t < ldp - 4 ? t : ldp - 4;
-#pragma unroll
-    for (int k = 0; k < RT; k++) p4[k] = *(const float4*)(pr + (size_t)k * rs + t);
-}
-
-// 4 keys of the tile: rows' p (already read), V from registers
-template <int RT>
-DEV void pvt_keys4(float (&acc)[RT][4], const float4 (&p4)[RT], const float4* v) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-        for (int k = 0; k < RT; k++) {
-            const float pk = j == 0 ? p4[k].x : j == 1 ? p4[k].y : j == 2 ? p4[k].z : p4[k].w;
-            acc[k][0] = fmaf(pk, v[j].x, acc[k][0]);
-            acc[k][1] = fmaf(pk, v[j].y, acc[k][1]);
-            acc[k][2] = fmaf(pk, v[j].z, acc[k][2]);
-            acc[k][3] = fmaf(pk, v[j].w, acc[k][3]);
-        }
-    }
-}
-
-template <int HD, int RT>
-__global__ __launch_bounds__(PVT_R * HD / (4 * RT)) void k_attn_pvt(const float* __restrict__ S, const float* __restrict__ vc,
-                                                         const int32_t* __restrict__ pos0p, int M, int n_q, int n_kv,
-                                                         int max_seq, int qt, int ldp, float* __restrict__ out,
-                                                         const uint8_t* __restrict__ o_sign, DpufPrep op) {
-    constexpr int R = PVT_R, NT = R * HD / (4 * RT), KV = PVT_KV;  // (R / RT) row groups x (HD / 4) dim groups
-    constexpr int NRG = R / RT;                                     // row groups
-    static_assert(R % (8 * RT) == 0 || R == 8 * RT, "whole row bands of 8 row groups");
-    constexpr int TPR = NT / R;  // threads per row in the softmax phases
-    extern __shared__ __align__(16) float P[];  // [R][ldp]
-    __shared__ float part[8 * R];
-    __shared__ float rowv[R][2];  // max, 1 / sum
-    // query tiles in dispatch order: the later (longer) half descending, then
-    // the earlier half ascending, so the two workgroups a CU takes together
-    // carry about the same number of keys
-    const int ny = gridDim.y, half = (ny + 1) / 2;
-    const int ty = (int)blockIdx.y < half ? ny - 1 - (int)blockIdx.y : (int)blockIdx.y - half;
-    const int kvh = blockIdx.x, m0 = ty * qt, tid = threadIdx.x;
-    const int lane = tid & 63, wv = tid >> 6;
-    const int G = n_q / n_kv;
-    const int pos0 = *pos0p;
-    const int mq = (m0 + qt < M ? m0 + qt : M) - m0;  // queries of this tile
-    auto row_len = [&](int r) { return r / G < mq ? pos0 + m0 + r / G + 1 : 0; };
-    const int Lmax = pos0 + m0 + mq, Lmin = pos0 + m0 + 1;
-    // score rows -> P (row r at r * ldp; 256 floats per wave instruction, ldp
-    // >= the rows' length rounded up to 256, so rows never overlap)
-    {
-        const int nch = (Lmax + 255) >> 8;
-        for (int u = wv; u < R * nch; u += NT / 64) {
-            const int r = u / nch, ch = u % nch;
-            const int rr = r / G < mq ? r : 0;
-            int t = 256 * ch + 4 * lane;
-            if (t + 3 >= max_seq) t = 0;
-            const float* src = S + ((size_t)(m0 + rr / G) * n_q + kvh * G + rr % G) * max_seq + t;
-            __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)(P + (size_t)r * ldp + 256 * ch), 16, 0,
-                                             0);
-        }
-    }
-    __syncthreads();
-    // row max: TPR consecutive threads per row, four running maxima each
-    {
-        const int r = tid / TPR, j = tid % TPR;
-        float m4[4] = {-1e30f, -1e30f, -1e30f, -1e30f};
-        const int L = row_len(r), L4 = L & ~3;
-        for (int t = 4 * j; t < L4; t += 4 * TPR) {
-            const float4 x = *(const float4*)&P[r * ldp + t];
-            m4[0] = fmaxf(m4[0], x.x);
-            m4[1] = fmaxf(m4[1], x.y);
-            m4[2] = fmaxf(m4[2], x.z);
-            m4[3] = fmaxf(m4[3], x.w);
-        }
-        if (j < L - L4) m4[0] = fmaxf(m4[0], P[r * ldp + L4 + j]);
-        float mx = fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]));
-#pragma unroll
-        for (int o = TPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-        if (j == 0) rowv[r][0] = mx;
-    }
-    __syncthreads();
-    // exp: the polynomial on t < kv_len & ~7 (float4 at a time), expf on the tail
-    {
-        const int n4w = ldp >> 2;
-        for (int e = tid; e < R * n4w; e += NT) {
-            const int r = e / n4w, c = e % n4w, n8 = row_len(r) & ~7;
-            if (4 * c >= n8) continue;
-            const float mx = rowv[r][0];
-            float4 x = *(float4*)&P[r * ldp + 4 * c];
-            x.x = exp_poly(x.x - mx);
-            x.y = exp_poly(x.y - mx);
-            x.z = exp_poly(x.z - mx);
-            x.w = exp_poly(x.w - mx);
-            *(float4*)&P[r * ldp + 4 * c] = x;
-        }
-        for (int e = tid; e < 8 * R; e += NT) {
-            const int r = e >> 3, L = row_len(r), t = (L & ~7) + (e & 7);
-            if (t < L) P[r * ldp + t] = expf_libc(P[r * ldp + t] - rowv[r][0]);
-        }
-    }
-    __syncthreads();
-    // the reference's eight sum lanes, each a chain over t = j (mod 8)
-    for (int e = tid; e < 8 * R; e += NT) {
-        const int r = e >> 3, j = e & 7;
-        part[e] = lds_sum_chain(P + r * ldp + j, 8, (row_len(r) & ~7) >> 3);
-    }
-    __syncthreads();
-    if (tid < R) {
-        const int L = row_len(tid), n8 = L & ~7;
-        float sp = hsum8(part + 8 * tid);
-        for (int t = n8; t < L; t++) sp += P[tid * ldp + t];
-        rowv[tid][1] = 1.0f / (sp + 1e-12f);
-    }
-    __syncthreads();
-    // p = e * inv, in place
-    {
-        const int n4w = ldp >> 2;
-        for (int e = tid; e < R * n4w; e += NT) {
-            const int r = e / n4w, c = e % n4w;
-            if (4 * c >= row_len(r)) continue;
-            const float inv = rowv[r][1];
-            float4 x = *(float4*)&P[r * ldp + 4 * c];
-            x.x = x.x * inv;
-            x.y = x.y * inv;
-            x.z = x.z * inv;
-            x.w = x.w * inv;
-            *(float4*)&P[r * ldp + 4 * c] = x;
-        }
-    }
-    __syncthreads();
-    // P.V: a wave holds 8 row groups x 8 dim groups, lane = 8 * (ri % 8) + di % 8
-    constexpr int WPR = HD / 32;  // waves per block of 8 row groups
-    const int ri = 8 * (wv / WPR) + (lane >> 3), di = 8 * (wv % WPR) + (lane & 7);
-    float acc[RT][4];
-#pragma unroll
-    for (int k = 0; k < RT; k++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[k][i] = 0.0f;
-    int Lr[RT];
-#pragma unroll
-    for (int k = 0; k < RT; k++) Lr[k] = row_len(ri + NRG * k);
-    // the thread's rows ri + 8k: the 8 row groups of a wave read rows ldp
-    // apart (ldp = 4 mod 64 words), on distinct banks; 4 consecutive rows per
-    // thread put them only 4 ldp apart, two to four groups per bank
-    const int rs = NRG * ldp;
-    const float* pr = P + (size_t)ri * ldp;
-    const float* vg = vc + (size_t)kvh * max_seq * HD + 4 * di;
-    // keys below Lmin, in whole batches, go to every row unconditionally
-    const int nfull = Lmin / KV * KV;
-    float4 va[KV], vb[KV];
-#pragma unroll
-    for (int j = 0; j < KV; j++) va[j] = *(const float4*)(vg + (size_t)(j < max_seq ? j : max_seq - 1) * HD);
-    int t0 = 0;
-    // (the scheduling barriers keep each batch's V loads ahead of the FMAs of
-    // the batch before it, and each 4 keys' p reads ahead of the FMAs of the 4
-    // keys before them, so their latencies are covered)
-    float4 pa[RT], pb[RT];
-    pvt_readp<RT>(pr, ldp, rs, 0, pa);
-    for (; t0 + 2 * KV <= nfull; t0 += 2 * KV) {
-#pragma unroll
-        for (int j = 0; j < KV; j++) {
-            const int t = t0 + KV + j;
-            vb[j] = *(const float4*)(vg + (size_t)(t < max_seq ? t : max_seq - 1) * HD);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < 2 * KV; j += 8) {
-            const float4* vv = j < KV ? va + j : vb + (j - KV);
-            pvt_readp<RT>(pr, ldp, rs, t0 + j + 4, pb);
-            __builtin_amdgcn_sched_barrier(0);
-            pvt_keys4<RT>(acc, pa, vv);
-            __builtin_amdgcn_sched_barrier(0);
-            pvt_readp<RT>(pr, ldp, rs, t0 + j + 8, pa);
-            __builtin_amdgcn_sched_barrier(0);
-            pvt_keys4<RT>(acc, pb, vv + 4);
-            __builtin_amdgcn_sched_barrier(0);
-            if (j + 8 == KV) {
-#pragma unroll
-                for (int jj = 0; jj < KV; jj++) {
-                    const int t = t0 + 2 * KV + jj;
-                    va[jj] = *(const float4*)(vg + (size_t)(t < max_seq ? t : max_seq - 1) * HD);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    }
-    if (t0 + KV <= nfull) {
-#pragma unroll
-        for (int j = 0; j < KV; j += 4) {
-            pvt_readp<RT>(pr, ldp, rs, t0 + j, pa);
-            pvt_keys4<RT>(acc, pa, va + j);
-        }
-        t0 += KV;
-    }
-    // the tile's last keys: row k takes key t only while t < its kv_len
-    for (int t = t0; t < Lmax; t++) {
-        const float4 v = *(const float4*)(vg + (size_t)t * HD);
-#pragma unroll
-        for (int k = 0; k < RT; k++) {
-            if (t < Lr[k]) {
-                const float pk = pr[(size_t)k * rs + t];
-                acc[k][0] = fmaf(pk, v.x, acc[k][0]);
-                acc[k][1] = fmaf(pk, v.y, acc[k][1]);
-                acc[k][2] = fmaf(pk, v.z, acc[k][2]);
-                acc[k][3] = fmaf(pk, v.w, acc[k][3]);
-            }
-        }
-    }
-    if (!op.q) {
-#pragma unroll
-        for (int k = 0; k < RT; k++) {
-            const int r = ri + NRG * k;
-            if (Lr[k] > 0)
-                *(float4*)(out + ((size_t)(m0 + r / G) * n_q + kvh * G + r % G) * HD + 4 * di) =
-                    make_float4(acc[k][0], acc[k][1], acc[k][2], acc[k][3]);
-        }
-        return;
-    }
-    // The prep of the O projection's input for the tile's rows (k_prep's
-    // arithmetic): the tile goes to LDS (over P, once every thread is done
-    // with it), then quad q = (row, 64-column block of the head) takes 16
-    // columns per lane through the signs, the FWHT-64 and the quantisation.
-    constexpr int LDT = HD + 4;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < RT; k++)
-        *(float4*)(P + (size_t)(ri + NRG * k) * LDT + 4 * di) = make_float4(acc[k][0], acc[k][1], acc[k][2], acc[k][3]);
-    __syncthreads();
-    const int qd = n_q * HD, nb = qd >> 5;
-    for (int qq = tid; qq < R * HD / 16; qq += NT) {  // quads of a row never straddle the loop's steps
-        const int bi = qq >> 2, qp = qq & 3, r = bi / (HD / 64), bh = bi % (HD / 64);
-        if (r / G >= mq) continue;  // whole quads
-        float v[16];
-        load16(P + (size_t)r * LDT + 64 * bh + 16 * qp, v);
-        const int m = m0 + r / G, blk = (kvh * G + r % G) * (HD / 64) + bh;
-        apply_sign_bits(v, quad_sign_bits(o_sign, blk, qp));
-        quad_fwht64(v, qp);
-        quad_quant_store(v, qp, blk, op.q + (size_t)m * qd, op.s + (size_t)m * nb, op.m + (size_t)m * nb,
-                         op.h ? op.h + (size_t)m * qd : nullptr);
-    }
-}
-
 __global__ __launch_bounds__(256) void k_attn(const float* __restrict__ q, const float* __restrict__ kc,
                                               const float* __restrict__ vc, float* __restrict__ out,
                                               float* __restrict__ scores, const int32_t* __restrict__ pos0p,
@@ -1116,34 +850,16 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     const int qt1 = 32 / G < M ? 32 / G : M;
     const dim3 g1(n_kv, (M + qt1 - 1) / qt1, (lmax + AS_KC - 1) / AS_KC);
     const size_t lds1 = (size_t)(AS_KC + 32) * (hd + 4) * 4;
-    // prefill with an even group: the register-tiled softmax + P.V kernel
-    if (M > 1 && (G & 1) == 0 && PVT_R % G == 0) {
-        const int ldp = 256 * ((lmax + 255) / 256) + 4;
-        const size_t ldst = (size_t)PVT_R * ldp * 4;
-        if (ldst <= 150 * 1024) {
-            const int qt = PVT_R / G;
-            const dim3 gt(n_kv, (M + qt - 1) / qt);
-            // the O input prep rides along when asked for (op.q set)
-            DpufPrep fop = op;
-            if (!prepped) fop.q = NULL;
+    const size_t budget = 112 * 1024;  // LDS bytes of a workgroup's probability rows
+    // several tokens, an even group of up to 16: the matrix-instruction
+    // kernels.  Less than one 16-row tile (M G < 16) over keys whose rows
+    // exceed the split kernels' LDS budget stays on the one-pair kernel.
+    if (M > 1 && (M * G >= 16 || (size_t)G * ((lmax + 7) & ~7) * 4 <= budget)) {
+        DpufPrep fop = op;
+        if (!prepped) fop.q = NULL;
+        if (attn_tile(s, M, lmax, q, kc, vc, NULL, out, scores, pos0p, n_q, n_kv, hd, max_seq, scale, o_sign, fop) ==
+            0) {
             if (fop.q) *prepped = 1;
-            if (hd == 64) {
-                hipLaunchKernelGGL(k_attn_sc<64>, g1, dim3(256), lds1, ST(s), q, kc, pos0p, M, n_q, n_kv, max_seq,
-                                   scale, qt1, scores);
-                hipLaunchKernelGGL((k_attn_pvt<64, PVT_RT>), gt, dim3(PVT_R * 64 / (4 * PVT_RT)), ldst, ST(s), scores, vc,
-                                   pos0p, M, n_q, n_kv, max_seq, qt, ldp, out, o_sign, fop);
-            } else if (hd == 128) {
-                hipLaunchKernelGGL(k_attn_sc<128>, g1, dim3(256), lds1, ST(s), q, kc, pos0p, M, n_q, n_kv, max_seq,
-                                   scale, qt1, scores);
-                hipLaunchKernelGGL((k_attn_pvt<128, PVT_RT>), gt, dim3(PVT_R * 128 / (4 * PVT_RT)), ldst, ST(s), scores, vc,
-                                   pos0p, M, n_q, n_kv, max_seq, qt, ldp, out, o_sign, fop);
-            } else {
-                hipLaunchKernelGGL(k_attn_sc<256>, g1, dim3(256), lds1, ST(s), q, kc, pos0p, M, n_q, n_kv, max_seq,
-                                   scale, qt1, scores);
-                hipLaunchKernelGGL((k_attn_pvt<256, PVT_RT>), gt, dim3(PVT_R * 256 / (4 * PVT_RT)), ldst, ST(s), scores, vc,
-                                   pos0p, M, n_q, n_kv, max_seq, qt, ldp, out, o_sign, fop);
-            }
-            LAUNCHED("k_attn_split_tiled");
             attn_path_note(0);
             return 0;
         }
@@ -1158,7 +874,6 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     // rows per workgroup keeps >= 32 dims per P.V chain group, so the
     // softmax each dim chunk repeats stays small next to P.V
     const int lcap = (lmax + 7) & ~7;
-    const size_t budget = 112 * 1024;
     int qt2 = 8 / G > 1 ? 8 / G : 1;
     if (qt2 > M) qt2 = M;
     while (qt2 > 1 && (size_t)qt2 * G * lcap * 4 > budget) qt2--;
@@ -1238,9 +953,20 @@ void dpuf_hip_attn(void* s, int32_t M, const float* q, const float* kc, const fl
 
 void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8 c8, float* out, float* scores,
                       const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq, float scale,
-                      const DpufWarm* warm) {
+                      const DpufWarm* warm, const uint8_t* o_sign, DpufPrep op, int32_t* prepped) {
     const int G = n_q / n_kv;
     if (lmax > max_seq) lmax = max_seq;
+    if (prepped) *prepped = 0;
+    if (M > 1) {
+        DpufPrep fop = op;
+        if (!prepped) fop.q = NULL;
+        if (attn_tile(s, M, lmax, q, NULL, NULL, &c8, out, scores, pos0, n_q, n_kv, hd, max_seq, scale, o_sign, fop) ==
+            0) {
+            if (fop.q) *prepped = 1;
+            attn_path_note(5);
+            return;
+        }
+    }
     const size_t lds1 = (size_t)G * hd * 4 + (size_t)Q8_SCK * hd + (size_t)Q8_SCK * (hd / 32) * 4;
     hipLaunchKernelGGL(k_attn_q8_sc, dim3(n_kv, (lmax + Q8_SCK - 1) / Q8_SCK, M), dim3(256), lds1, ST(s), q, c8,
                        scores, pos0, n_q, n_kv, hd, max_seq, scale);

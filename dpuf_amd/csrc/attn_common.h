@@ -276,6 +276,14 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
 int32_t attn_wide_q8(void* s, int32_t lmax, const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd,
                      int32_t max_seq, float* scores, float* out, DpufKvQ8 c8, const DpufWarm* wm);
 
+// The attention of M > 1 tokens on the fp32 matrix instructions
+// (attn_tile.hip), even groups of up to 16 heads, over the fp32 cache (kc, vc)
+// or, with c8 set, the int8 cache; op.q set: the O projection's input prep in
+// place of out.  -1 (nothing launched) when the shape does not take it.
+int32_t attn_tile(void* s, int32_t M, int32_t lmax, const float* q, const float* kc, const float* vc,
+                  const DpufKvQ8* c8, float* out, float* scores, const int32_t* pos0, int32_t n_q, int32_t n_kv,
+                  int32_t hd, int32_t max_seq, float scale, const uint8_t* o_sign, DpufPrep op);
+
 // Warm-up workgroup i (of wm.n_wg; grid position L, so XCD L % 8): the
 // units of its XCD are (job j, round lg, the k-th workgroup of job j on that
 // XCD), job by job; it takes a share of at most WARM_MAXU of them, puts their

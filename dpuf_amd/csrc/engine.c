@@ -624,7 +624,7 @@ DPUF_EXPORT void* dpuf_engine_create(const DpufModelConfig* cfg, const DpufLayer
         e->gate = (float*)dpuf_hip_malloc(B * e->I * 4);
         e->up = (float*)dpuf_hip_malloc(B * e->I * 4);
         e->logits = (float*)dpuf_hip_malloc(B * (size_t)e->V * 4);
-        e->scores = (float*)dpuf_hip_malloc(B * (size_t)e->nq * e->max_seq * 4);
+        e->scores = (float*)dpuf_hip_malloc(B * (size_t)e->nq * ((size_t)e->max_seq + DPUF_HIP_ATTN_SLOTS) * 4);
         e->embeds = (float*)dpuf_hip_malloc(B * e->H * 4);
         for (int i = 0; i < 3; i++) {
             e->prep[i].q = (int8_t*)dpuf_hip_malloc(B * maxd);
@@ -914,7 +914,10 @@ static void enqueue_ms_attention(Engine* e, int32_t l, int32_t M, float eps, flo
             const DpufKvQ8 c8 = slot_q8(e, e->ms_slot[m], l);
             dpuf_hip_qk_rope_kv(s, 1, q, k, v, qn, kn, eps, e->d_cos, e->d_sin, NULL, NULL, pp, e->nq, e->nkv, e->hd,
                                 e->max_seq, &c8);
-            dpuf_hip_attn_q8(s, 1, keys, q, c8, ao, e->scores, pp, e->nq, e->nkv, e->hd, e->max_seq, scale, NULL);
+            DpufPrep none;
+            memset(&none, 0, sizeof none);
+            dpuf_hip_attn_q8(s, 1, keys, q, c8, ao, e->scores, pp, e->nq, e->nkv, e->hd, e->max_seq, scale, NULL,
+                             NULL, none, NULL);
             continue;
         }
         float* kc = slot_k(e, e->ms_slot[m]) + lo;
@@ -995,9 +998,11 @@ static void enqueue_layers(Engine* e, int32_t M, int32_t keep_tiles) {
                 dpuf_hip_qk_rope_kv(s, M, e->q, e->k, e->v, e->d_norm[4 * l + 1], e->d_norm[4 * l + 2], eps,
                                     e->d_cos, e->d_sin, NULL, NULL, e->d_pos0, e->nq, e->nkv, e->hd, e->max_seq, &c8);
                 const DpufWarm wq = attn_warm_fed_o(e, &lj, ln);
+                int32_t prepped = 0;
                 dpuf_hip_attn_q8(s, M, e->capturing ? e->cap_lmax : e->host_pos0 + M, e->q, c8, e->ao, e->scores,
-                                 e->d_pos0, e->nq, e->nkv, e->hd, e->max_seq, scale, M == 1 ? &wq : NULL);
-                if (M > 1) dpuf_hip_prep(s, M, e->qd, e->ao, W[W_O].sign, e->prep[0]);
+                                 e->d_pos0, e->nq, e->nkv, e->hd, e->max_seq, scale, M == 1 ? &wq : NULL,
+                                 W[W_O].sign, e->prep[0], &prepped);
+                if (M > 1 && !prepped) dpuf_hip_prep(s, M, e->qd, e->ao, W[W_O].sign, e->prep[0]);
                 o_prep = M == 1;
                 fused = 1;
             } else if (M == 1 && e->host_pos0 + 1 <= ATT_SPLIT_MIN)

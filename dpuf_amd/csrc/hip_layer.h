@@ -206,6 +206,9 @@ void dpuf_hip_qk_rope_kv(void* s, int32_t M, float* q, float* k, const float* v,
 void dpuf_hip_attn(void* s, int32_t M, const float* q, const float* kc, const float* vc, float* out,
                    float* scores, const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd,
                    int32_t max_seq, float scale);
+/* Attention scratch of M tokens (the `scores` arguments): n_q rows of max_seq
+ * scores per token, then per row the score maxima of this many key ranges. */
+#define DPUF_HIP_ATTN_SLOTS 64
 /* Split attention (scores kernel + softmax/P.V kernel) over keys up to
  * lmax; -1 (nothing launched) when the shape does not fit.  With op.q and
  * prepped set, a launch that can also writes the O projection's input prep
@@ -225,10 +228,11 @@ int32_t dpuf_hip_attn_decode_rope(void* s, int32_t lmax, float* q, const float* 
                                   int32_t n_kv, int32_t hd, int32_t max_seq, float scale, const DpufWarm* warm);
 /* Attention over the int8 KV cache (kv_type 1) for M tokens at positions
  * pos0 .. pos0 + M - 1 of one layer; lmax bounds the keys any replay reaches.
- * warm (or NULL): as for dpuf_hip_attn_decode_rope, on the one-token path. */
+ * warm (or NULL): as for dpuf_hip_attn_decode_rope, on the one-token path.
+ * o_sign, op, prepped: as for dpuf_hip_attn_split. */
 void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8 c8, float* out, float* scores,
                       const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq, float scale,
-                      const DpufWarm* warm);
+                      const DpufWarm* warm, const uint8_t* o_sign, DpufPrep op, int32_t* prepped);
 /* n rows of fp32 K and V (device) quantised into rows row0 .. of the int8
  * cache, as the KV store does; and n values from element off dequantised. */
 void dpuf_hip_q8_rows(void* s, const float* k, const float* v, int32_t n, int32_t hd, DpufKvQ8 c8, size_t row0);
