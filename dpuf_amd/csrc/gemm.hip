@@ -588,6 +588,23 @@ DEV float sk_round_chain(float acc, const float (&d)[SKP_RS], const uint32_t (&w
     return acc;
 }
 
+// The same for the 64-block pairs of modes 13 / 14 (dpuf_avx2.c:2871-2882): fd
+// is fma(float(D0), xs0, float(D1) * xs1), wv the pair's fp16 (d, m), xm its
+// xm_s, and np the pairs of the round:
+//   acc = fma(fd, d, acc); acc = fma(m, xm_s, acc)
+DEV float sk_round_chain_asym(float acc, const float (&fd)[SKP_RS / 2], const uint32_t (&wv)[SKP_RS / 2],
+                              const gm_f4 (&xm)[SKP_RS / 8], int np) {
+#pragma unroll
+    for (int j = 0; j < SKP_RS / 2; j++) {
+        const gm_h2 hw = __builtin_bit_cast(gm_h2, wv[j]);
+        if (j < np) {  // uniform
+            acc = __builtin_fmaf(fd[j], (float)hw[0], acc);
+            acc = __builtin_fmaf((float)hw[1], xm[j >> 2][j & 3], acc);
+        }
+    }
+    return acc;
+}
+
 // Polls an LDS counter until it reaches want, at most 2^22 polls (false when
 // it ran out); the polled value is wave-uniform, so the loop is scalar.
 DEV bool sk_wait(uint32_t* p, uint32_t want) {
@@ -601,10 +618,60 @@ DEV bool sk_wait(uint32_t* p, uint32_t want) {
     return true;
 }
 
+// Scales and sums of the two 64-blocks b0, b0 + 2 of a token (pairs clamped
+// into the row; n_blk is even in modes 13 / 14).
+DEV void sk_xs_load(__amdgpu_buffer_rsrc_t rs, __amdgpu_buffer_rsrc_t rm, int xt, int b0, int n_blk, gm_u4& xs,
+                    gm_u4& xm) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const uint32_t o = (uint32_t)(4 * (xt + min(b0 + 2 * p, n_blk - 2)));
+        const gm_u2 a = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
+        const gm_u2 b = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rm, o, 0, 0));
+        xs[2 * p] = a[0];
+        xs[2 * p + 1] = a[1];
+        xm[2 * p] = b[0];
+        xm[2 * p + 1] = b[1];
+    }
+}
+
+// Modes 13 / 14: a producer wave's two 64-block pairs of a round.  tw / th are
+// the transposed nibble and high-bit words of its 4 blocks, xs / xm the lane's
+// token scales and sums of them; fd of each pair goes to LDS in place of the
+// two D tiles (half the traffic, and the chains' products with xs are taken
+// off them) and the lanes of kc 0 store the pairs' xm_s.
+DEV void sk_pairs(const uint32_t (&tw)[4], const uint32_t (&th)[4], const gm_u4 (&ax)[SKP_RB], gm_u4 xs, gm_u4 xm,
+                  float (*dq)[4][64], float* xml, int l) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        // through scalars: this compiler's bit cast of a vector element reads element 0
+        const uint32_t s0 = xs[2 * p], s1 = xs[2 * p + 1];
+        const float xs0 = __builtin_bit_cast(float, s0), xs1 = __builtin_bit_cast(float, s1);
+        const gm_f4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gm_unpack_a_asym(tw[2 * p], th[2 * p]),
+                                                               __builtin_bit_cast(gm_h8, ax[2 * p]),
+                                                               (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        const gm_f4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(gm_unpack_a_asym(tw[2 * p + 1], th[2 * p + 1]),
+                                                               __builtin_bit_cast(gm_h8, ax[2 * p + 1]),
+                                                               (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const float p1 = d1[v] * xs1;
+            dq[p][v][l] = fmaf(d0[v], xs0, p1);
+        }
+        const float pa = (float)(int32_t)xm[2 * p] * xs0, pb = (float)(int32_t)xm[2 * p + 1] * xs1;
+        if (l < 16) xml[p] = (pa + pb) * 0.125f;
+    }
+}
+
+// Modes 13 / 14 on this kernel against one wave per 16 rows of k_gemm_mfma
+// (which a 4-token pass leaves bound by one stage's load latency at a time):
+// down [12288 -> 4096] in mode 14 at M = 4, 41 MB, 103.7 -> 20.4 us.
+template <int MODE>
 __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
-    __shared__ __align__(16) float dq[SK_NB][SKP_RS][4][64];    // D tiles [buf][block][v][lane]
+    constexpr bool ASYM = MODE != 12;
+    constexpr int ND = ASYM ? SKP_RS / 2 : SKP_RS;              // tiles handed over per round
+    __shared__ __align__(16) float dq[SK_NB][ND][4][64];        // D (fd of a pair) tiles [buf][block][v][lane]
     __shared__ __align__(16) uint16_t wsl[SK_NB][16][SKP_RS];   // weight scales [buf][row][block]
-    __shared__ __align__(16) float xsl[SK_NB][16][SKP_RS + 4];  // token scales [buf][token][block], rows padded
+    __shared__ __align__(16) float xsl[SK_NB][16][ND + 4];      // token scales (xm_s of a pair) [buf][token][block], rows padded
     // hand-off counters per buffer, cumulative: full[b] counts producer waves
     // done with a round in b, freed[b] chain waves done reading one
     __shared__ uint32_t full[SK_NB], freed[SK_NB];
@@ -628,9 +695,10 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
     const GmJob& J = ji == 0 ? A.j[0] : ji == 1 ? A.j[1] : A.j[2];
     const uint16_t* const Jh = ji == 0 ? A.j[0].h : ji == 1 ? A.j[1].h : A.j[2].h;
     const float* const Js = ji == 0 ? A.j[0].s : ji == 1 ? A.j[1].s : A.j[2].s;
+    const int32_t* const Jm = ji == 0 ? A.j[0].m : ji == 1 ? A.j[1].m : A.j[2].m;
     const int gf = J.g0 + 2 * (fr - A.tb[ji]);  // first group of the fragment
     const int K = A.K, n_blk = K >> 5, n_r = (n_blk + SKP_RS - 1) / SKP_RS;
-    const size_t gstride = (size_t)n_blk * 144;
+    const size_t gstride = (size_t)n_blk * (MODE == 14 ? 208 : 144);
     const int i16 = l & 15, kc = l >> 4;
     if (tid < SK_NB) {
         full[tid] = 0;
@@ -649,16 +717,23 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
         const uint32_t on = (uint32_t)((size_t)(ga - gf) * gstride + (size_t)n_blk * 16 + (i16 & 7) * 16);
         const int sj = (l >> 2) & 3, sd = l & 3, sg = min(gf + ((l >> 4) & 1), J.g1 - 1);
         const uint32_t os = (uint32_t)((size_t)(sg - gf) * gstride + sd * 4);
+        // mode 14: the row's 8 bytes of high bits of block b0 + kc
+        const uint32_t oh = (uint32_t)((size_t)(ga - gf) * gstride + (size_t)n_blk * 144 + (i16 & 7) * 8);
+        const __amdgpu_buffer_rsrc_t rm =
+            __builtin_amdgcn_make_buffer_rsrc(ASYM ? (void*)Jm : (void*)Js, 0, M * n_blk * 4, GM_RSRC3);
         const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc((void*)Jh, 0, M * K * 2, GM_RSRC3);
         const uint32_t ho = (uint32_t)(2 * (min(i16, M - 1) * K + 8 * kc));
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)Js, 0, M * n_blk * 4, GM_RSRC3);
         const int xt = min(i16, M - 1) * n_blk;
         uint32_t wq[SK_P][4], wsq[SK_P];
         gm_u4 ax[SK_P][SKP_RB];
-        float xsq[SK_P];
+        gm_u4 xsq[SK_P], xmq[SK_P];  // mode 12: xsq[..][0] is block b0 + kc's scale; else blocks b0 .. b0 + 3
+        uint32_t hq[SK_P][2];
         // weights, scales and activations of round r in one ring slot (the
         // wait counter retires loads in issue order)
-        auto load = [&](int r, uint32_t (&q)[4], uint32_t& sq, gm_u4 (&a)[SKP_RB], float& x) {
+        auto load = [&](int r, int u) {
+            uint32_t(&q)[4] = wq[u];
+            gm_u4(&a)[SKP_RB] = ax[u];
             const int b0 = r * SKP_RS + w * SKP_RB;
             const gm_u4 v = __builtin_bit_cast(
                 gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rw, on + (uint32_t)min(b0 + kc, n_blk - 1) * 128u, 0, 0));
@@ -666,23 +741,32 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
             q[1] = v[1];
             q[2] = v[2];
             q[3] = v[3];
-            sq = __builtin_amdgcn_raw_buffer_load_b32(rw, os + (uint32_t)min(b0 + sj, n_blk - 1) * 16u, 0, 0);
+            if (MODE == 14) {
+                const gm_u2 h = __builtin_bit_cast(
+                    gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rw, oh + (uint32_t)min(b0 + kc, n_blk - 1) * 64u, 0, 0));
+                hq[u][0] = h[0];
+                hq[u][1] = h[1];
+            }
+            wsq[u] = __builtin_amdgcn_raw_buffer_load_b32(rw, os + (uint32_t)min(b0 + sj, n_blk - 1) * 16u, 0, 0);
 #pragma unroll
             for (int j = 0; j < SKP_RB; j++)
                 a[j] = __builtin_bit_cast(gm_u4,
                                           __builtin_amdgcn_raw_buffer_load_b128(rh, ho, min(b0 + j, n_blk - 1) * 64, 0));
-            x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                              rs, (uint32_t)(4 * (xt + min(b0 + kc, n_blk - 1))), 0, 0));
+            if (ASYM)
+                sk_xs_load(rs, rm, xt, b0, n_blk, xsq[u], xmq[u]);
+            else
+                xsq[u][0] =
+                    __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)(4 * (xt + min(b0 + kc, n_blk - 1))), 0, 0);
         };
 #pragma unroll
-        for (int u = 0; u < SK_P - 1; u++) load(u, wq[u], wsq[u], ax[u], xsq[u]);
+        for (int u = 0; u < SK_P - 1; u++) load(u, u);
         for (int it0 = 0; it0 < n_r; it0 += SK_P) {
 #pragma unroll
             for (int u = 0; u < SK_P; u++) {
                 const int it = it0 + u;
                 if (it >= n_r) break;  // uniform
                 const int un = (u + SK_P - 1) % SK_P;
-                load(it + SK_P - 1, wq[un], wsq[un], ax[un], xsq[un]);
+                load(it + SK_P - 1, un);
                 {
                     // round it goes to buffer it % SK_NB once the chains have
                     // read round it - SK_NB from it
@@ -694,20 +778,34 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
                     uint32_t t0 = wq[u][0], t1 = wq[u][1], t2 = wq[u][2], t3 = wq[u][3];
                     skp_transpose(t0, t1, t2, t3);
                     const uint32_t tw[4] = {t0, t1, t2, t3};
+                    if (ASYM) {
+                        uint32_t th[4] = {0u, 0u, 0u, 0u};
+                        if (MODE == 14) {
+                            // word kc / 2 of the row's high bits, the odd chunk's in the upper nibbles
+                            th[0] = hq[u][0];
+                            th[1] = hq[u][0] >> 4;
+                            th[2] = hq[u][1];
+                            th[3] = hq[u][1] >> 4;
+                            skp_transpose(th[0], th[1], th[2], th[3]);
+                        }
+                        sk_pairs(tw, th, ax[u], xsq[u], xmq[u],
+                                 &dq[buf][2 * w], &xsl[buf][i16][2 * w], l);
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < SKP_RB; j++) {
-                        const gm_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            gm_unpack_a(tw[j]), __builtin_bit_cast(gm_h8, ax[u][j]),
-                            (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        for (int j = 0; j < SKP_RB; j++) {
+                            const gm_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                gm_unpack_a(tw[j]), __builtin_bit_cast(gm_h8, ax[u][j]),
+                                (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
-                        for (int v = 0; v < 4; v++) dq[buf][w * SKP_RB + j][v][l] = d[v];
+                            for (int v = 0; v < 4; v++) dq[buf][w * SKP_RB + j][v][l] = d[v];
+                        }
                     }
                     if (l < 32) {
                         const int row = ((l >> 4) & 1) * 8 + 2 * sd;
                         wsl[buf][row][w * SKP_RB + sj] = (uint16_t)(wsq[u] & 0xFFFFu);
                         wsl[buf][row + 1][w * SKP_RB + sj] = (uint16_t)(wsq[u] >> 16);
                     }
-                    xsl[buf][i16][w * SKP_RB + kc] = xsq[u];
+                    if (!ASYM) xsl[buf][i16][w * SKP_RB + kc] = __builtin_bit_cast(float, xsq[u][0]);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                     if (l == 0) __hip_atomic_fetch_add(&full[buf], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
@@ -726,9 +824,9 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
             if (!sk_wait(&full[buf], (uint32_t)(SK_NP * ((it - 1) / SK_NB + 1))) && l == 0) atomicOr(A.err, 1);
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
             const int nj = min(SKP_RS, n_blk - b0);  // uniform
-            float d[SKP_RS];
+            float d[ND];
 #pragma unroll
-            for (int j = 0; j < SKP_RS; j++) d[j] = dq[buf][j][c][l];
+            for (int j = 0; j < ND; j++) d[j] = dq[buf][j][c][l];
             // scale words as separate 32-bit values (see k_gemm_skp)
             uint32_t wv[SKP_RS / 2];
 #pragma unroll
@@ -739,10 +837,13 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
                 wv[4 * q + 2] = t[2];
                 wv[4 * q + 3] = t[3];
             }
-            gm_f4 xr[SKP_RS / 4];
+            gm_f4 xr[ND / 4];
 #pragma unroll
-            for (int q = 0; q < SKP_RS / 4; q++) xr[q] = *(const gm_f4*)&xsl[buf][i16][4 * q];
-            acc = sk_round_chain(acc, d, wv, xr, nj);
+            for (int q = 0; q < ND / 4; q++) xr[q] = *(const gm_f4*)&xsl[buf][i16][4 * q];
+            if constexpr (ASYM)
+                acc = sk_round_chain_asym(acc, d, wv, xr, nj >> 1);
+            else
+                acc = sk_round_chain(acc, d, wv, xr, nj);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
             if (l == 0) __hip_atomic_fetch_add(&freed[buf], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
@@ -770,12 +871,14 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_sk(GmArgs A) {
 // turns that into the MFMA A layout: word kc of each of the 4 blocks in lane
 // (i, kc).
 // ---------------------------------------------------------------------------
-template <int NR>
+template <int NR, int MODE>
 __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
+    constexpr bool ASYM = MODE != 12;
+    constexpr int ND = ASYM ? SKP_RS / 2 : SKP_RS;  // tiles handed over per round
     static_assert(SKP_P % NR == 0 && NR <= 4, "ring depth must be a multiple of the rounds per fragment");
-    __shared__ __align__(16) float dq[2][SKP_RS][4][64];    // D tiles [buf][block][v][lane]
+    __shared__ __align__(16) float dq[2][ND][4][64];        // D (fd of a pair) tiles [buf][block][v][lane]
     __shared__ __align__(16) uint16_t wsl[2][16][SKP_RS];   // weight scales [buf][row][block]
-    __shared__ __align__(16) float xsl[2][16][SKP_RS + 4];  // token scales [buf][token][block], rows padded
+    __shared__ __align__(16) float xsl[2][16][ND + 4];      // token scales (xm_s of a pair) [buf][token][block], rows padded
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
     const int M = A.M, bid = blockIdx.x;
     if (bid >= A.tb[A.n_jobs]) {
@@ -793,11 +896,12 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
     const GmJob& J = ji == 0 ? A.j[0] : ji == 1 ? A.j[1] : A.j[2];
     const uint16_t* const Jh = ji == 0 ? A.j[0].h : ji == 1 ? A.j[1].h : A.j[2].h;
     const float* const Js = ji == 0 ? A.j[0].s : ji == 1 ? A.j[1].s : A.j[2].s;
+    const int32_t* const Jm = ji == 0 ? A.j[0].m : ji == 1 ? A.j[1].m : A.j[2].m;
     const int lb = bid - A.tb[ji], nwg = A.tb[ji + 1] - A.tb[ji];
     const int nf = (J.g1 - J.g0 + 1) >> 1;              // fragments of the job
     const int n_my = (nf - lb + nwg - 1) / nwg;         // >= 1: nwg <= nf
     const int K = A.K, n_blk = K >> 5, S = n_my * NR;   // steps: NR rounds per fragment
-    const uint32_t gstride = (uint32_t)n_blk * 144u;    // J.g1 gstride < 2^32 is checked at launch
+    const uint32_t gstride = (uint32_t)n_blk * (MODE == 14 ? 208u : 144u);    // J.g1 gstride < 2^32 is checked at launch
     const int i16 = l & 15, kc = l >> 4;
 
     if (w < SK_NP) {
@@ -814,13 +918,19 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
         // fragment, block (l >> 2) & 3 of the wave, rows 2 (l & 3), 2 (l & 3) + 1
         const int sj = (l >> 2) & 3, sd = l & 3;
         const bool os_hi = ((l >> 4) & 1) != 0;
+        const uint32_t oh = (uint32_t)n_blk * 144u + (i16 & 7) * 8;  // mode 14: the row's 8 bytes of high bits
         uint32_t wq[SKP_P][4], wsq[SKP_P];
+        uint32_t hq[SKP_P][2];
         gm_u4 ax[NR][SKP_RB];
-        float xh[NR];  // token l & 15, block l >> 4 of the wave, per round
+        // token l & 15, per round: mode 12 block l >> 4 of the wave's scale in
+        // [0], else the wave's 4 blocks' scales and sums
+        gm_u4 xh[NR], xhm[NR];
         {
             const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc((void*)Jh, 0, M * K * 2, GM_RSRC3);
             const __amdgpu_buffer_rsrc_t rs =
                 __builtin_amdgcn_make_buffer_rsrc((void*)Js, 0, M * n_blk * 4, GM_RSRC3);
+            const __amdgpu_buffer_rsrc_t rm =
+                __builtin_amdgcn_make_buffer_rsrc(ASYM ? (void*)Jm : (void*)Js, 0, M * n_blk * 4, GM_RSRC3);
             const uint32_t ho = (uint32_t)(2 * (min(i16, M - 1) * K + 8 * kc));
             const int xt = min(i16, M - 1) * n_blk;
 #pragma unroll
@@ -830,14 +940,19 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
                 for (int j = 0; j < SKP_RB; j++)
                     ax[r][j] = __builtin_bit_cast(
                         gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rh, ho, min(b0 + j, n_blk - 1) * 64, 0));
-                const uint32_t xo = (uint32_t)(4 * (xt + min(b0 + kc, n_blk - 1)));
-                xh[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, xo, 0, 0));
+                if (ASYM) {
+                    sk_xs_load(rs, rm, xt, b0, n_blk, xh[r], xhm[r]);
+                } else {
+                    const uint32_t xo = (uint32_t)(4 * (xt + min(b0 + kc, n_blk - 1)));
+                    xh[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, xo, 0, 0);
+                }
             }
         }
         // loads of step s = NR fl + r: fragment lb + fl nwg, round r.  Steps
         // past the workgroup's last fragment re-read that fragment.
         const int fr_last = lb + (n_my - 1) * nwg;
-        auto wload = [&](int fl, int r, uint32_t (&q)[4], uint32_t& sq) {
+        auto wload = [&](int fl, int r, int u) {
+            uint32_t(&q)[4] = wq[u];
             const int fr = min(lb + fl * nwg, fr_last);
             const uint32_t gb = (uint32_t)(J.g0 + 2 * fr) * gstride;
             const uint32_t g2 = J.g0 + 2 * fr + 1 < J.g1 ? gstride : 0u;  // uniform
@@ -849,37 +964,57 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
             q[2] = v[2];
             q[3] = v[3];
             const uint32_t vos = (os_hi ? g2 : 0u) + (uint32_t)min(b0 + sj, n_blk - 1) * 16u + sd * 4;
-            sq = __builtin_amdgcn_raw_buffer_load_b32(rw, vos, gb, 0);
+            wsq[u] = __builtin_amdgcn_raw_buffer_load_b32(rw, vos, gb, 0);
+            if (MODE == 14) {
+                const uint32_t voh = oh + (on_hi ? g2 : 0u) + (uint32_t)min(b0 + kc, n_blk - 1) * 64u;
+                const gm_u2 h = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rw, voh, gb, 0));
+                hq[u][0] = h[0];
+                hq[u][1] = h[1];
+            }
         };
 #pragma unroll
-        for (int u = 0; u < SKP_P - 1; u++) wload(u / NR, u % NR, wq[u], wsq[u]);
+        for (int u = 0; u < SKP_P - 1; u++) wload(u / NR, u % NR, u);
         for (int it0 = 0; it0 <= S; it0 += SKP_P) {
 #pragma unroll
             for (int u = 0; u < SKP_P; u++) {
                 const int it = it0 + u;
                 if (it > S) break;  // uniform
                 const int un = (u + SKP_P - 1) % SKP_P;
-                wload((it0 + u + SKP_P - 1) / NR, un % NR, wq[un], wsq[un]);
+                wload((it0 + u + SKP_P - 1) / NR, un % NR, un);
                 const int r = u % NR;
                 if (it < S && r * SKP_RS < n_blk) {
                     const int buf = u & 1;
                     uint32_t t0 = wq[u][0], t1 = wq[u][1], t2 = wq[u][2], t3 = wq[u][3];
                     skp_transpose(t0, t1, t2, t3);
                     const uint32_t tw[4] = {t0, t1, t2, t3};
+                    if (ASYM) {
+                        uint32_t th[4] = {0u, 0u, 0u, 0u};
+                        if (MODE == 14) {
+                            // word kc / 2 of the row's high bits, the odd chunk's in the upper nibbles
+                            th[0] = hq[u][0];
+                            th[1] = hq[u][0] >> 4;
+                            th[2] = hq[u][1];
+                            th[3] = hq[u][1] >> 4;
+                            skp_transpose(th[0], th[1], th[2], th[3]);
+                        }
+                        sk_pairs(tw, th, ax[r], xh[r], xhm[r],
+                                 &dq[buf][2 * w], &xsl[buf][i16][2 * w], l);
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < SKP_RB; j++) {
-                        const gm_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            gm_unpack_a(tw[j]), __builtin_bit_cast(gm_h8, ax[r][j]),
-                            (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        for (int j = 0; j < SKP_RB; j++) {
+                            const gm_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                gm_unpack_a(tw[j]), __builtin_bit_cast(gm_h8, ax[r][j]),
+                                (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
-                        for (int v = 0; v < 4; v++) dq[buf][w * SKP_RB + j][v][l] = d[v];
+                            for (int v = 0; v < 4; v++) dq[buf][w * SKP_RB + j][v][l] = d[v];
+                        }
                     }
                     if (l < 32) {
                         const int row = ((l >> 4) & 1) * 8 + 2 * sd;
                         wsl[buf][row][w * SKP_RB + sj] = (uint16_t)(wsq[u] & 0xFFFFu);
                         wsl[buf][row + 1][w * SKP_RB + sj] = (uint16_t)(wsq[u] >> 16);
                     }
-                    xsl[buf][i16][w * SKP_RB + kc] = xh[r];
+                    if (!ASYM) xsl[buf][i16][w * SKP_RB + kc] = __builtin_bit_cast(float, xh[r][0]);
                 }
                 __syncthreads();
             }
@@ -902,9 +1037,9 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
                 const int buf = (u + 1) & 1, b0 = r * SKP_RS;
                 const int nj = min(SKP_RS, n_blk - b0);  // uniform, <= 0 past the last round
                 if (nj > 0) {
-                    float d[SKP_RS];
+                    float d[ND];
 #pragma unroll
-                    for (int j = 0; j < SKP_RS; j++) d[j] = dq[buf][j][c][l];
+                    for (int j = 0; j < ND; j++) d[j] = dq[buf][j][c][l];
                     // the scale words as separate 32-bit values: this compiler
                     // selected the wrong register for words 1..3 when they
                     // went from a 4 x 32-bit vector into v_fma_mix_f32
@@ -917,10 +1052,13 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
                         wv[4 * q + 2] = t[2];
                         wv[4 * q + 3] = t[3];
                     }
-                    gm_f4 xr[SKP_RS / 4];
+                    gm_f4 xr[ND / 4];
 #pragma unroll
-                    for (int q = 0; q < SKP_RS / 4; q++) xr[q] = *(const gm_f4*)&xsl[buf][i16][4 * q];
-                    acc = sk_round_chain(acc, d, wv, xr, nj);
+                    for (int q = 0; q < ND / 4; q++) xr[q] = *(const gm_f4*)&xsl[buf][i16][4 * q];
+                    if constexpr (ASYM)
+                        acc = sk_round_chain_asym(acc, d, wv, xr, nj >> 1);
+                    else
+                        acc = sk_round_chain(acc, d, wv, xr, nj);
                 }
                 if (r == NR - 1) {
                     const int fr = lb + fl * nwg;
@@ -943,8 +1081,8 @@ typedef void (*GmKernel)(GmArgs);
 // Workgroups of a K-split GEMM instance the device holds at once.
 static int gm_capacity(GmKernel k, int threads) {
     static int n_cu = 0;
-    static GmKernel c_k[4];
-    static int c_cap[4], c_n = 0;
+    static GmKernel c_k[9];
+    static int c_cap[9], c_n = 0;
     for (int i = 0; i < c_n; i++)
         if (c_k[i] == k) return c_cap[i];
     if (n_cu == 0) {
@@ -957,13 +1095,20 @@ static int gm_capacity(GmKernel k, int threads) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, 0) != hipSuccess || per_cu <= 0)
         per_cu = 1;
     const int cap = per_cu * n_cu;
-    if (c_n < 4) {
+    if (c_n < 9) {
         c_k[c_n] = k;
         c_cap[c_n++] = cap;
     }
     return cap;
 }
 
+
+extern "C++" {
+template <int MODE>
+static GmKernel gm_skp_of(int nr) {
+    return nr == 1 ? k_gemm_skp<1, MODE> : nr == 2 ? k_gemm_skp<2, MODE> : k_gemm_skp<4, MODE>;
+}
+}
 
 // Gate and up of M > 16 tokens with the SwiGLU + dead zone + prep of the down
 // input in the same launch (k_gemm_mfma<..., true>): a workgroup's
@@ -1067,11 +1212,14 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
         const int mode = jobs[0].w.mode;  // one mode per launch (dpuf_hip_gemv groups them)
         long long gmax = 0;
         for (int i = 0; i < n_jobs; i++) gmax = gmax > jobs[i].g1 ? gmax : jobs[i].g1;
-        if (mode == 12 && M <= 16 && n_blk <= 128 && gmax * n_blk * 144 < 0xFFFFFFFFll) {
+        // up to 16 tokens, every mode: K-split (modes 13 / 14 at M = 4 and the 8B
+        // shapes: Q or O 34.0 -> 10.6 us, K + V 36.8 -> 11.1, down 103.7 -> 20.4
+        // against k_gemm_mfma, whose waves are then one per 16 rows)
+        if (M <= 16 && n_blk <= 128 && gmax * n_blk * dpuf_grp_unit(mode) < 0xFFFFFFFFll) {
             // one 16-token tile, K <= 4096: persistent K-split workgroups,
             // each job's share of the chip in proportion to its fragments
             const int NR = n_blk <= 32 ? 1 : n_blk <= 64 ? 2 : 4;
-            GmKernel k = NR == 1 ? k_gemm_skp<1> : NR == 2 ? k_gemm_skp<2> : k_gemm_skp<4>;
+            GmKernel k = mode == 13 ? gm_skp_of<13>(NR) : mode == 14 ? gm_skp_of<14>(NR) : gm_skp_of<12>(NR);
             int cap = gm_capacity(k, 64 * (SK_NP + SK_NC));
             if (dpuf_hip_mv_max_wg() > 0 && cap > dpuf_hip_mv_max_wg()) cap = dpuf_hip_mv_max_wg();
             int nfr[3], ftot = 0;
@@ -1092,7 +1240,7 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
             LAUNCHED("k_gemm_skp");
             return;
         }
-        if (mode == 12 && M <= 16) {
+        if (M <= 16) {
             // one 16-token tile: the K-split kernel, one workgroup per 16 rows
             int f = 0;
             for (int i = 0; i < n_jobs; i++) {
@@ -1106,7 +1254,7 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
                 note(hipErrorInvalidValue, "dpuf_hip_gemv: no device error word bound");
                 return;
             }
-            hipLaunchKernelGGL(k_gemm_sk, dim3(f + G.zt), dim3(64 * (SK_NP + SK_NC)), 0, ST(s), G);
+            hipLaunchKernelGGL(mode == 13 ? k_gemm_sk<13> : mode == 14 ? k_gemm_sk<14> : k_gemm_sk<12>, dim3(f + G.zt), dim3(64 * (SK_NP + SK_NC)), 0, ST(s), G);
             LAUNCHED("k_gemm_sk");
             return;
         }
@@ -1114,8 +1262,6 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
         const int gx = (t + G.zt + 7) & ~7;
         G.gy = (M + 16 * GM_TT - 1) / (16 * GM_TT);
         const dim3 grid = GM_XCD ? dim3(gx * G.gy) : dim3(gx, G.gy);
-        // modes 13 / 14 take this kernel at every M (the K-split kernels
-        // are mode 12 only)
         if (mode == 13)
             hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 13, 4>), grid, dim3(256), 0, ST(s), G);
         else if (mode == 14)

@@ -51,6 +51,21 @@ def test_matmul_bit_exact(eng, orc, mode, rows, cols, m):
 
 
 @pytest.mark.parametrize("mode", [13, 14])
+@pytest.mark.parametrize("rows,cols,m", [(16, 64, 2), (40, 1088, 16), (24, 2112, 9), (200, 4032, 5), (8216, 4096, 4),
+                                         (40, 4160, 16), (72, 8256, 2), (200, 12288, 7)])
+def test_few_token_split_k(eng, orc, mode, rows, cols, m):
+    """2..16 tokens (the K-split kernels): one 64-block, rounds and waves'
+    shares that end early, an odd group count, several fragments per
+    workgroup, and K above 4 096; bit for bit as every other M."""
+    blob, d = _mat(rows, cols, 3 + rows + mode, mode)
+    x = np.random.default_rng(rows + cols + m).standard_normal((m, cols)).astype(np.float32)
+    x[m - 1, 32:64] = 1e-6
+    log(f"mode {mode} rows={rows} cols={cols} M={m}")
+    g, o = _run(eng, orc, d, x)
+    assert bits_equal(g, o), maxdiff(g, o)
+
+
+@pytest.mark.parametrize("mode", [13, 14])
 @pytest.mark.parametrize("rows,cols", [(1024, 4096), (4096, 12288), (12288, 4096), (4096, 4096)])
 def test_matmul_8b_shapes_m1(eng, orc, mode, rows, cols):
     """The Qwen3-8B GEMV shapes (K/V, down, gate/up, Q/O) at M = 1."""
