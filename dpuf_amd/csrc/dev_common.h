@@ -532,6 +532,8 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // Vector types of the MFMA kernels.
 typedef _Float16 gm_h8 __attribute__((ext_vector_type(8)));
 typedef float gm_f4 __attribute__((ext_vector_type(4)));
+typedef int32_t gm_i16 __attribute__((ext_vector_type(16)));
+typedef int32_t gm_i4 __attribute__((ext_vector_type(4)));
 typedef uint32_t gm_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t gm_u4 __attribute__((ext_vector_type(4)));
 

@@ -21,50 +21,59 @@
 #include "dev_common.h"
 #include "hip_internal.h"
 
-// M > 1 GEMM on the matrix cores (slab path, dpuf_avx2.c:2643-2676).
+// M > 16 GEMM on the matrix cores (slab path, dpuf_avx2.c:2643-2676): k_gemm_mfma
+// (16 x 16 tiles) and k_gemm_x32 (32 x 32 tiles).
 //
 // For every (row, token) the reference accumulates every block:
 //   acc = fma(float(D - sum8), fp16(ws) * xs, acc), blocks ascending,
-// with D the u4 x i8 dot of the block and sum8 = 8 * sum(q).  Since
-// D - sum8 = sum((u - 8) * q) exactly, one v_mfma_f32_16x16x32_f16 per block
-// with A = (u - 8) and B = q, both exact in f16, gives float(D - sum8) for a
-// 16-row x 16-token tile (every partial sum is an integer below 2^15, exact
-// in the fp32 accumulator).  The epilogue is the reference's two rounded
-// operations, sp = ws * xs and the fma, with the chains in registers across
-// the block loop, so the block order is the reference's.
+// with D the u4 x i8 dot of the block and sum8 = 8 * sum(q).  D - sum8 =
+// sum((u - 8) * q), so one int8 MFMA per block and tile gives it exactly; the
+// epilogue is the reference's two rounded operations with the chains in
+// registers across the block loop, so the block order is the reference's.
 //
-// A workgroup of NW = 4 or 8 waves computes 16 NW GM_RF rows x 16 TT tokens;
-// wave w owns GM_RF 16-row fragments and all the tokens as TT 16-token tiles
-// (GM_RF TT MFMAs per block).  With 8 waves twice the rows share a staged
-// token tile: half the activation staging per MFMA.  Activations arrive as fp16 (DpufPrep.h, written by the
-// prep kernels) and are staged in LDS, GM_SB blocks per stage, double-
-// buffered, one barrier per stage; a token's 64 bytes per block are four
-// 16-byte chunks stored XOR-swizzled by token so a fragment read is free of
-// bank conflicts.  A block's fragments are read from LDS one block ahead of
-// its MFMAs.  Weights, nibbles and scales, are read straight into registers
-// one stage ahead.  MFMA lane layouts (gfx950, checked on the device): A lane
-// l = row l % 16, k = 8 (l / 16) + e; B lane l = token l % 16, same k; D lane
-// l = token l % 16, rows 4 (l / 16) + v.
+// What bounds both is instructions per tile and block (the chains leave 12
+// per 256 outputs that no matrix instruction can take) and, in order in a
+// wave, the latencies between them.  So:
+//   * A = 16 (u - 8), one v_bitop3 per 4 nibbles (the nibble's top bit
+//     flipped, in a byte's upper half), 3 instructions per nibble word where
+//     u - 8 as fp16 took 11;
+//   * the MFMA's C is the bit pattern 0x3e22f983 (1 / (2 pi)) in every
+//     element: |16 (D - sum8)| < 2^20 stays inside that binade, so the result
+//     read as a float is 1 / (2 pi) + n 2^-26 exactly and one exact
+//     subtraction gives n 2^-26 at full rate (v_cvt_f32_i32 issues at half);
+//   * weight scales are widened to float once per workgroup when they are
+//     staged, so the product with xs is a v_mul_f32 (v_fma_mix_f32 issues at
+//     half rate).
+// acc carries the factor 2^-22 (modes 13 / 14, whose u needs no offset:
+// 2^-26), removed at the end: powers of two commute with every rounding here
+// as long as no partial sum is below 2^-104 in magnitude.
+//
+// Activations (int8, token scales) and weight scales are staged in LDS a
+// stage of several blocks at a time, double-buffered, one barrier per stage.
+// LDS rows of a block are padded so that the staging writes of consecutive
+// blocks fall into different banks (unpadded: 8-way conflicts).  Weight
+// nibbles are read straight into a register ring several quads ahead, 16
+// bytes per lane, and exchanged between the wave's lane rows into the MFMA
+// layout.  MFMA lane layouts (gfx950, checked on the device): 16x16x32: A / B
+// lane l = row / token l % 16, k = 8 (l / 16) + e; D lane l = token l % 16,
+// rows 4 (l / 16) + v.  32x32x32: A / B lane l = row l % 32, k = 16 (l / 32) +
+// e; D lane l = column l % 32, rows 8 (v / 4) + 4 (l / 32) + v % 4.
+//
+// us per launch at the 8B widths, before (one 16-row x 64-token fp16 tile per
+// wave for every M) -> now: down M = 29 85 -> 32, M = 90 93 -> 43, M = 512 144
+// -> 119; O 30 -> 13, 31 -> 17, 47.5 -> 38; mode 14 down M = 90 135 -> 51, M =
+// 512 223 -> 146; gate + up with the SwiGLU M = 29 46 -> 32, M = 512 204 -> 178.
 // ---------------------------------------------------------------------------
-#define GM_SB 4  // blocks per LDS stage
-#define GM_RF 1  // 16-row fragments per wave (workgroup = 64 GM_RF rows)
-#define GM_TT 4  // 16-token tiles per workgroup
-#define GM_XCD 1  // XCD-grouped workgroup order
-// Launches of at least this many rows (the fused gate + up projection) and
-// more than GM_NW8_MINM tokens take 8-wave workgroups: pp512 at the 8B shape
-// 21.2 -> 20.85 ms, pp256 13.2 -> 13.0 ms, pp128 10.2 -> 10.5 ms (half the
-// workgroups of the 4-wave grid leave CUs idle), pp32 and pp64 unchanged;
-// Q/K/V, O and down on 8 waves as well, pp512 21.1 ms; down as well, 20.8 ms.
-#define GM_NW8_ROWS 16384
-#define GM_NW8_MINM 128
 
+#define GM_SWI_ROWS 16384  // gate + up rows from which the fused SwiGLU launch pays
 #define GM_RSRC3 0x00020000  // buffer descriptor word 3 (gfx9 family): 32-bit raw data
 
 struct GmJob {
     const uint8_t* g;  // dense groups of the matrix
     int g0, g1;        // groups computed
     int rows;
-    const uint16_t* h;  // activations as fp16 [M][K]
+    const uint16_t* h;  // activations as fp16 [M][K] (K-split kernels)
+    const int8_t* q;    // activations as int8 [M][K]
     const float* s;     // block scales [M][K/32]
     const int32_t* m;   // 8 * block sums of q [M][K/32] (modes 13 / 14)
     float* out;        // out[m * ldo + row]
@@ -117,52 +126,54 @@ DEV gm_h8 gm_unpack_a_asym(uint32_t w, uint32_t h) {
 }
 
 
-// Modes 13 / 14 hold a 64-block's even half (its D tiles, token scales and
-// sums, row scales) across the odd one: 2 waves per SIMD keep that in
-// registers instead of spilling at the 128 VGPRs of 4.
-template <int TT, int RF, int MODE, int NW, bool SWI = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MODE == 12 ? 4 : 2))) void k_gemm_mfma(
-    GmArgs A) {
-    constexpr int NT = 16 * TT;  // tokens per workgroup
-    constexpr int NTH = 64 * NW;  // threads per workgroup
-    constexpr int GPW = 2 * RF * NW;  // 8-row groups per workgroup
+// ---------------------------------------------------------------------------
+// k_gemm_mfma: NW waves of 16 rows each, TT 16-token tiles per workgroup, for
+// launches with few tiles: a wave of one tile (TT = 1) leaves the most waves,
+// and a tile's serial chain over K is then all of the launch's length.
+template <int TT, int MODE, int NW, bool SWI>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : TT == 1 || (MODE != 12 && TT == 4) ? 2 : 3))) void
+k_gemm_mfma(GmArgs A) {
+    constexpr int NT = 16 * TT;              // tokens per workgroup
+    constexpr int NTH = 64 * NW;             // threads per workgroup
+    constexpr int GPW = 2 * NW;              // 8-row groups per workgroup
+    constexpr int SB = 32 / TT;              // blocks per LDS stage
+    constexpr int QS = SB / 4;               // 4-block quads per stage
+    constexpr int PF = TT == 1 ? 8 : 4;      // quads of nibbles in flight
+    constexpr int G = TT == 1 ? 4 : TT == 2 ? 2 : 1;  // blocks per LDS read set
+    constexpr int NX = NT * SB;              // token scales per stage (512)
     constexpr bool ASYM = MODE != 12;
-    static_assert(GM_SB % 2 == 0, "a stage holds whole 64-blocks");
+    constexpr uint32_t BASE = 0x3e22f983u;   // 1 / (2 pi)
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    static_assert(!SWI || (NW == 8 && RF == 1 && TT == 4 && MODE == 12), "the SwiGLU pairing: 4 + 4 waves");
-    __shared__ __align__(16) uint8_t bq[2][GM_SB][NT][64];  // f16 activations [stage][block][token][k]
-    __shared__ __align__(16) float bs[2][GM_SB][16][TT];    // block scales [stage][block][token % 16][token / 16]
-    __shared__ __align__(16) int32_t bm[ASYM ? 2 : 1][GM_SB][16][TT];  // 8 * block sums (modes 13 / 14)
-    __shared__ __align__(16) uint32_t bw[2][GM_SB][4 * GPW];  // weight scales [stage][block][group * 4 + word]
+    static_assert((2 * QS) % PF == 0, "ring slots are static over two stages");
+    static_assert(!SWI || (NW == 8 && MODE == 12), "the SwiGLU pairing: 4 + 4 waves");
+    __shared__ __align__(16) uint8_t bq[2][SB][NT * 32 + 32];          // int8 activations [stage][block][token][k]
+    __shared__ __align__(16) float bs[2][NT][SB + 4];            // token scales [stage][token][block], rows padded
+    __shared__ __align__(16) float bm[ASYM ? 2 : 1][NT][SB / 2 + 4];  // xm_s of the 64-blocks (modes 13 / 14)
+    __shared__ __align__(16) float bw[2][SB][GPW * 8 + 8];           // weight scales [stage][block][row]
     // Workgroups go to the 8 XCDs round-robin by linear id L.  L = xcd +
     // 8 j with j = gy r + ty puts row tile 8 r + xcd of every token tile ty on
     // one XCD, dispatched back to back, so the gy workgroups that read the
     // same weights run together and share them through that XCD's L2.
-#if GM_XCD
     const int jx = blockIdx.x >> 3, ty = jx % A.gy;
     const int rt = (jx / A.gy) * 8 + (blockIdx.x & 7);
-#else
-    const int rt = blockIdx.x, ty = blockIdx.y;
-#endif
     if (rt >= A.tb[A.n_jobs]) {
         // zeroing tiles, then padding of the grid (whole workgroups)
         const int zi = rt - A.tb[A.n_jobs];
         if (zi < A.zt) {
             const int r = A.z0 + 64 * zi + (threadIdx.x & 63);
-            for (int t = threadIdx.x >> 6; t < 16 * TT; t += NW) {
-                const int m = ty * 16 * TT + t;
+            for (int t = threadIdx.x >> 6; t < NT; t += NW) {
+                const int m = ty * NT + t;
                 if (m < A.M && r < A.z1) A.zo[(size_t)m * A.zld + r] = 0.0f;
             }
         }
         return;
     }
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, i16 = l & 15, kc = l >> 4;
-    const int wu = __builtin_amdgcn_readfirstlane(w);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i16 = l & 15, kc = l >> 4;
     // SWI: waves 0-3 compute job 0 (gate), waves 4-7 job 1 (up), the same 64
     // rows (8 groups) of each, and the activations are the jobs' shared input
     int ji = 0;
     if (SWI) {
-        ji = wu >> 2;
+        ji = w >> 2;
     } else {
         if (A.n_jobs > 1 && rt >= A.tb[1]) ji = 1;
         if (A.n_jobs > 2 && rt >= A.tb[2]) ji = 2;
@@ -170,329 +181,306 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MODE ==
     // the job's fields picked from the kernel arguments by uniform selects,
     // so they stay in scalar registers through the loop
     const GmJob& J = ji == 0 ? A.j[0] : ji == 1 ? A.j[1] : A.j[2];
-    const uint16_t* const Jh = ji == 0 ? A.j[0].h : ji == 1 ? A.j[1].h : A.j[2].h;
+    const int8_t* const Jq = ji == 0 ? A.j[0].q : ji == 1 ? A.j[1].q : A.j[2].q;
     const float* const Js = ji == 0 ? A.j[0].s : ji == 1 ? A.j[1].s : A.j[2].s;
     const int32_t* const Jm = ji == 0 ? A.j[0].m : ji == 1 ? A.j[1].m : A.j[2].m;
     // first group of the workgroup (SWI: of the wave's job), and the wave's
     // place among the waves of that job
     const int gb = SWI ? J.g0 + rt * (GPW / 2) : J.g0 + (rt - A.tb[ji]) * GPW;
-    const int wl = SWI ? (wu & 3) : wu;
+    const int wl = SWI ? (w & 3) : w;
     const int m0 = ty * NT;
-    const int K = A.K, M = A.M, n_blk = K >> 5;
+    const int K = A.K, M = A.M, n_blk = K >> 5, n_st = (n_blk + SB - 1) / SB;
     const size_t gstride = (size_t)n_blk * (MODE == 14 ? 208 : 144);
 
-    // Every load is a buffer load: a wave-uniform descriptor, a 32-bit lane
-    // offset fixed for the launch and a scalar block offset, so addressing
-    // costs no vector instructions in the loop (and a load past a
-    // descriptor's range reads 0 instead of faulting).  Weights of the
-    // wave's RF fragments (groups clamped into the job) are addressed from
-    // the wave's first group.
-    const int gw0 = min(gb + 2 * RF * wl, J.g1 - 1);
-    const size_t wbytes = (size_t)(J.g1 - gw0) * gstride;
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(J.g + (size_t)gw0 * gstride), 0, (int)(wbytes < 0xFFFFFFFFu ? wbytes : 0xFFFFFFFFu), GM_RSRC3);
-    uint32_t on[RF], oh[RF];
-#pragma unroll
-    for (int f = 0; f < RF; f++) {
-        const int ga = min(gb + 2 * RF * wl + 2 * f + (i16 >> 3), J.g1 - 1);
-        on[f] = (uint32_t)((size_t)(ga - gw0) * gstride + (size_t)n_blk * 16 + (i16 & 7) * 16 + kc * 4);
-        // mode 14: the lane's high-bit word (chunk kc's bits are in word kc / 2)
-        oh[f] = (uint32_t)((size_t)(ga - gw0) * gstride + (size_t)n_blk * 144 + (i16 & 7) * 8 + (kc >> 1) * 4);
-    }
-    // Weight scales go through LDS with the activations: a stage's GPW
-    // groups x GM_SB blocks x 8 fp16 scales are WD dwords, dword d = (tid +
-    // NTH k) % WD (group d / (4 GM_SB), block (d / 4) % GM_SB, word d % 4),
-    // addressed from the workgroup's first group; threads past WD repeat a
-    // dword.  Blocks past the end read bytes that are never used.
-    // SWI: groups 0-7 of a stage are job 0's, 8-15 job 1's; with one dword
-    // per thread (d = tid % 256) a wave's dwords are all of one job.
-    constexpr int WD = 4 * GPW * GM_SB, WPT = (WD + NTH - 1) / NTH;
-    static_assert(!SWI || (WPT == 1 && WD == 256), "one job per wave's scale dwords");
-    const int jg = SWI ? (wu & 3) >> 1 : ji;
-    const GmJob& JG = jg == 0 ? A.j[0] : jg == 1 ? A.j[1] : A.j[2];
+    // Every load is a buffer load with its whole offset in the lane: past the
+    // descriptor's range it reads 0, and what lies in range past a row's or a
+    // group's last block is never computed, so no load has a clamp or a
+    // branch around it.  Rows and tokens are clamped once.
+    const auto rsrc = [](const void* p, size_t n) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(n < 0xFFFFFFFFu ? n : 0xFFFFFFFFu), GM_RSRC3);
+    };
+    const int gw0 = min(gb + 2 * wl, J.g1 - 1);
+    const __amdgpu_buffer_rsrc_t rw = rsrc(J.g + (size_t)gw0 * gstride, (size_t)(J.g1 - gw0) * gstride);
+    const int ga = min(gb + 2 * wl + (i16 >> 3), J.g1 - 1);
+    // nibbles: lane (row i16, kc) reads the row's 16 bytes of block 4 q + kc;
+    // mode 14: its 8 bytes of high bits of that block
+    const uint32_t on = (uint32_t)((size_t)(ga - gw0) * gstride + (size_t)n_blk * 16 + (i16 & 7) * 16 + kc * 128);
+    const uint32_t oh = (uint32_t)((size_t)(ga - gw0) * gstride + (size_t)n_blk * 144 + (i16 & 7) * 8 + kc * 64);
+    gm_u4 wn[PF];
+    gm_u2 wh[PF];
+    auto wload = [&](int q, int slot) {
+        wn[slot] = __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rw, on + (uint32_t)q * 512u, 0, 0));
+        if (MODE == 14)
+            wh[slot] = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rw, oh + (uint32_t)q * 256u, 0, 0));
+    };
+    // Staging.  16-byte piece c = tid + NTH k: token c / (2 SB), half c & 1 of
+    // block (c / 2) % SB, so consecutive threads read a token's contiguous
+    // bytes.  Scale i = tid + NTH k: token i / SB, block i % SB (modes 13 / 14
+    // pair i: its two scales and sums).  Weight scales: 16 bytes per (group,
+    // block), group-major, addressed from the workgroup's first group (SWI:
+    // groups 0-7 are job 0's, 8-15 job 1's, a whole wave in one job).
+    constexpr int CPT = 2 * NX / NTH, SPT = (ASYM ? NX / 2 : NX) / NTH > 0 ? (ASYM ? NX / 2 : NX) / NTH : 1;
+    static_assert(2 * NX % NTH == 0 && (!ASYM || NX / 2 % NTH == 0) && NX % NTH == 0, "whole shares per thread");
+    constexpr int WS = GPW * SB;
+    static_assert(WS <= NTH && WS % 64 == 0, "at most one weight scale piece per thread");
+    const int jg = SWI ? (tid % WS) / (WS / 2) : ji;
+    const int jgu = SWI ? __builtin_amdgcn_readfirstlane(jg) : ji;
+    const GmJob& JG = jgu == 0 ? A.j[0] : jgu == 1 ? A.j[1] : A.j[2];
     const int gbg = SWI ? JG.g0 + rt * (GPW / 2) : gb;
-    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(JG.g + (size_t)gbg * gstride), 0,
-        (int)((size_t)(JG.g1 - gbg) * gstride < 0xFFFFFFFFu ? (size_t)(JG.g1 - gbg) * gstride : 0xFFFFFFFFu),
-        GM_RSRC3);
-    uint32_t og[WPT], sw[WPT];  // load offsets; the thread's scale dwords of the stage in flight
-    int wgi[WPT];               // their LDS word index in a stage buffer
-#pragma unroll
-    for (int k = 0; k < WPT; k++) {
-        const int wd = (tid + NTH * k) % WD, g = wd / (4 * GM_SB), b = (wd >> 2) % GM_SB, w4 = wd & 3;
-        const int gj = SWI ? (g & (GPW / 2 - 1)) : g;  // the group within its job's rows
-        og[k] = (uint32_t)((size_t)(min(gbg + gj, JG.g1 - 1) - gbg) * gstride + b * 16 + w4 * 4);
-        wgi[k] = b * 4 * GPW + g * 4 + w4;
-    }
-    // staging: a stage holds NT tokens x GM_SB blocks of 64 fp16 bytes, four
-    // 16-byte chunks each.  Chunk c = tid + NTH k of the stage is chunk c & 3
-    // of pair c / 4 = (token (c / 4) % NT, block (c / 4) / NT), so the 64
-    // lanes of a load read 16 tokens' 64 contiguous bytes.  Scale i = tid +
-    // NTH k is pair i.  Loads are unconditional, at token and block clamped
-    // into range: a token past M only feeds output columns that are never
-    // stored, a block past the end is never computed, and a load without a
-    // branch around it keeps the compiler's wait counts exact.
-    constexpr int CPT = NT * GM_SB * 4 / NTH, SPT = (NT * GM_SB + NTH - 1) / NTH;
-    static_assert(CPT >= 1 && NT * GM_SB * 4 % NTH == 0, "whole chunks per thread");
-    const int n_st = (n_blk + GM_SB - 1) / GM_SB;
-    gm_u4 sq[CPT];  // a native vector: a struct copy would keep the array in scratch
-    float ss[SPT];
-    int32_t sm[SPT];
-    // byte offsets of the token rows (M K < 2^30 is checked at launch); with
-    // NT = 64 a chunk's block (wave / 4 + NW k / 4) and a scale's block (the
-    // wave, + NW k) are uniform and go into the scalar offset
-    const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc((void*)Jh, 0, M * K * 2, GM_RSRC3);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)Js, 0, M * n_blk * 4, GM_RSRC3);
-    const __amdgpu_buffer_rsrc_t rm =
-        __builtin_amdgcn_make_buffer_rsrc(ASYM ? (void*)Jm : (void*)Js, 0, M * n_blk * 4, GM_RSRC3);
-    uint32_t ho[CPT], so[SPT];
+    const __amdgpu_buffer_rsrc_t rg = rsrc(JG.g + (size_t)gbg * gstride, (size_t)(JG.g1 - gbg) * gstride);
+    const int wg = (tid % WS) / SB, wb = tid % SB;
+    const uint32_t og = (uint32_t)((size_t)(min(gbg + (SWI ? (wg & 7) : wg), JG.g1 - 1) - gbg) * gstride + wb * 16);
+    const __amdgpu_buffer_rsrc_t rq = rsrc(Jq, (size_t)M * K);
+    const __amdgpu_buffer_rsrc_t rs = rsrc(Js, (size_t)M * n_blk * 4);
+    const __amdgpu_buffer_rsrc_t rm = rsrc(ASYM ? (const void*)Jm : (const void*)Js, (size_t)M * n_blk * 4);
+    gm_u4 sq[CPT];
+    float ss[SPT][2];
+    int32_t sm[SPT][2];
+    gm_u4 sw;
+    uint32_t qo[CPT], so[SPT];
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
-        const int pr = (tid >> 2) + (NTH / 4) * k, m = min(m0 + pr % NT, M - 1);
-        const int sbt = NT == 64 ? 0 : pr / NT;
-        ho[k] = (uint32_t)(2 * (m * K + 32 * sbt + 8 * (tid & 3)));
+        const int c = tid + NTH * k;
+        qo[k] = (uint32_t)(min(m0 + c / (2 * SB), M - 1) * K + 16 * (c % (2 * SB)));
     }
 #pragma unroll
     for (int k = 0; k < SPT; k++) {
-        const int i = min(tid + NTH * k, NT * GM_SB - 1), m = min(m0 + i % NT, M - 1);
-        const int sbt = NT == 64 ? 0 : i / NT;
-        so[k] = (uint32_t)(4 * (m * n_blk + sbt));
+        const int i = tid + NTH * k;
+        so[k] = ASYM ? (uint32_t)(4 * (min(m0 + i / (SB / 2), M - 1) * n_blk + 2 * (i % (SB / 2))))
+                     : (uint32_t)(4 * (min(m0 + i / SB, M - 1) * n_blk + i % SB));
     }
-    // the stage's first block, clamped so that a stage's blocks stay in range
-    // when it starts in range (blocks past the end are never computed)
     auto stage_load = [&](int st) {
 #pragma unroll
-        for (int k = 0; k < CPT; k++) {
-            const int sbt = NT == 64 ? (wu >> 2) + k * (NW / 4) : 0;
-            const int b = NT == 64 ? min(st * GM_SB + sbt, n_blk - 1) : st * GM_SB;
-            sq[k] = __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rh, ho[k], b * 64, 0));
-        }
+        for (int k = 0; k < CPT; k++)
+            sq[k] = __builtin_bit_cast(gm_u4,
+                                       __builtin_amdgcn_raw_buffer_load_b128(rq, qo[k] + (uint32_t)st * (SB * 32u), 0, 0));
 #pragma unroll
         for (int k = 0; k < SPT; k++) {
-            const int b = NT == 64 ? min(st * GM_SB + wu + NW * k, n_blk - 1) : st * GM_SB;
-            ss[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, so[k], b * 4, 0));
-            if (ASYM) sm[k] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rm, so[k], b * 4, 0);
+            const uint32_t o = so[k] + (uint32_t)st * (SB * 4u);
+            if (ASYM) {
+                const gm_u2 a = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
+                const gm_u2 b = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rm, o, 0, 0));
+                const uint32_t a0 = a[0], a1 = a[1];
+                ss[k][0] = __builtin_bit_cast(float, a0);
+                ss[k][1] = __builtin_bit_cast(float, a1);
+                sm[k][0] = (int32_t)b[0];
+                sm[k][1] = (int32_t)b[1];
+            } else {
+                const uint32_t a = __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0);
+                ss[k][0] = __builtin_bit_cast(float, a);
+            }
         }
-#pragma unroll
-        for (int k = 0; k < WPT; k++) sw[k] = __builtin_amdgcn_raw_buffer_load_b32(rg, og[k], st * GM_SB * 16, 0);
+        sw = __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rg, og + (uint32_t)st * (SB * 16u), 0, 0));
     };
     auto stage_store = [&](int buf) {
 #pragma unroll
         for (int k = 0; k < CPT; k++) {
-            const int c = tid + NTH * k, pr = c >> 2, tk = pr % NT, sbt = pr / NT, qu = c & 3;
-            *(gm_u4*)&bq[buf][sbt][tk][16 * (qu ^ ((tk >> 1) & 3))] = sq[k];
+            const int c = tid + NTH * k;
+            *(gm_u4*)&bq[buf][(c >> 1) % SB][32 * (c / (2 * SB)) + 16 * (c & 1)] = sq[k];
         }
 #pragma unroll
         for (int k = 0; k < SPT; k++) {
-            const int i = tid + NTH * k, tk = i % NT, sbt = i / NT;
-            if (NT * GM_SB % NTH == 0 || i < NT * GM_SB) {
-                bs[buf][sbt][tk & 15][tk >> 4] = ss[k];
-                if (ASYM) bm[ASYM ? buf : 0][sbt][tk & 15][tk >> 4] = sm[k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < WPT; k++) (&bw[buf][0][0])[wgi[k]] = sw[k];
-    };
-    // nibble words (and mode 14 high-bit words) of one stage, per fragment and block
-    uint32_t wn[2][GM_SB][RF];
-    uint32_t wh[2][GM_SB][RF];
-    auto weights_load = [&](int st, uint32_t (&n)[GM_SB][RF], uint32_t (&hn)[GM_SB][RF]) {
-#pragma unroll
-        for (int sb = 0; sb < GM_SB; sb++) {
-            const int b = min(st * GM_SB + sb, n_blk - 1);
-#pragma unroll
-            for (int f = 0; f < RF; f++) {
-                n[sb][f] = __builtin_amdgcn_raw_buffer_load_b32(rw, on[f], b * 128, 0);
-                hn[sb][f] = MODE == 14 ? __builtin_amdgcn_raw_buffer_load_b32(rw, oh[f], b * 64, 0) : 0u;
-            }
-        }
-    };
-
-    gm_f4 acc[RF][TT];
-#pragma unroll
-    for (int f = 0; f < RF; f++)
-#pragma unroll
-        for (int t = 0; t < TT; t++) acc[f][t] = (gm_f4){0.0f, 0.0f, 0.0f, 0.0f};
-
-    // B fragments, token scales and the lane's 4 row scales of one block,
-    // read from LDS one block ahead of its MFMAs so the read latency hides
-    // behind the block before.  The row scales stay two separate 32-bit
-    // words: this compiler selected the first word's register for both
-    // words' fp16 halves when they came as one 2 x 32-bit vector into
-    // v_fma_mix_f32.
-    gm_h8 bfr[2][TT];
-    float xsr[2][TT];
-    int32_t xmr[2][TT];
-    uint32_t wsr[2][RF][2];
-    auto lds_b = [&](int buf, int sb, int slot) {
-#pragma unroll
-        for (int f = 0; f < RF; f++) {
-            const int e = (2 * (RF * wu + f) + (kc >> 1)) * 4 + (kc & 1) * 2;
-            wsr[slot][f][0] = bw[buf][sb][e];
-            wsr[slot][f][1] = bw[buf][sb][e + 1];
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t++) xsr[slot][t] = bs[buf][sb][i16][t];
-        if (ASYM) {
-#pragma unroll
-            for (int t = 0; t < TT; t++) xmr[slot][t] = bm[ASYM ? buf : 0][sb][i16][t];
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const int tok = 16 * t + i16;
-            bfr[slot][t] = *(const gm_h8*)&bq[buf][sb][tok][16 * (kc ^ ((tok >> 1) & 3))];
-        }
-    };
-    // modes 13 / 14: the even block of a 64-block pair waits in registers for
-    // the odd one: its D tiles, token scales and sums, and the lane's 4 d
-    gm_f4 dk[RF][TT];
-    float xs0k[TT];
-    int32_t xm0k[TT];
-    float dsk[RF][4];
-    auto compute = [&](int st, int buf, const uint32_t (&n)[GM_SB][RF], const uint32_t (&hn)[GM_SB][RF]) {
-        lds_b(buf, 0, 0);
-#pragma unroll
-        for (int sb = 0; sb < GM_SB; sb++) {
-            if (st * GM_SB + sb >= n_blk) break;  // uniform
-            if (sb + 1 < GM_SB) lds_b(buf, sb + 1, (sb + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-            gm_h8 a[RF];
-            _Float16 wsh[RF][4];
-#pragma unroll
-            for (int f = 0; f < RF; f++) {
-                a[f] = ASYM ? gm_unpack_a_asym(n[sb][f], (hn[sb][f] >> ((kc & 1) * 4)))
-                            : gm_unpack_a(n[sb][f]);
-                const gm_h2 lo = __builtin_bit_cast(gm_h2, wsr[sb & 1][f][0]),
-                            hi = __builtin_bit_cast(gm_h2, wsr[sb & 1][f][1]);
-                wsh[f][0] = lo[0];
-                wsh[f][1] = lo[1];
-                wsh[f][2] = hi[0];
-                wsh[f][3] = hi[1];
-            }
-            float xs[TT];
-#pragma unroll
-            for (int t = 0; t < TT; t++) xs[t] = xsr[sb & 1][t];
+            const int i = tid + NTH * k;
             if (ASYM) {
-                // 64-block epilogue (dpuf_avx2.c:2871-2882), rows 4 kc' + v
-                // of the fragment for token 16 t + i16:
-                //   fdot = fma(float(D0), xs0, float(D1) * xs1)
-                //   acc = fma(fdot, d, acc); acc = fma(m, xm_s, acc)
-                if ((sb & 1) == 0) {
-#pragma unroll
-                    for (int t = 0; t < TT; t++) {
-                        xs0k[t] = xs[t];
-                        xm0k[t] = xmr[sb & 1][t];
-#pragma unroll
-                        for (int f = 0; f < RF; f++)
-                            dk[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[f], bfr[sb & 1][t],
-                                                                              (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int f = 0; f < RF; f++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) dsk[f][v] = (float)wsh[f][v];
-                } else {
-#pragma unroll
-                    for (int t = 0; t < TT; t++) {
-                        const float pa = (float)xm0k[t] * xs0k[t], pb = (float)xmr[sb & 1][t] * xs[t];
-                        const float xms = (pa + pb) * 0.125f;
-#pragma unroll
-                        for (int f = 0; f < RF; f++) {
-                            const gm_f4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                a[f], bfr[sb & 1][t], (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                            for (int v = 0; v < 4; v++) {
-                                const float p1 = d1[v] * xs[t];
-                                const float fd = fmaf(dk[f][t][v], xs0k[t], p1);
-                                acc[f][t][v] = fmaf(fd, dsk[f][v], acc[f][t][v]);
-                                acc[f][t][v] = fmaf((float)wsh[f][v], xms, acc[f][t][v]);
-                            }
-                        }
-                    }
-                }
-                continue;
+                const int t = i / (SB / 2), p = i % (SB / 2);
+                bs[buf][t][2 * p] = ss[k][0];
+                bs[buf][t][2 * p + 1] = ss[k][1];
+                const float pa = (float)sm[k][0] * ss[k][0], pb = (float)sm[k][1] * ss[k][1];
+                bm[ASYM ? buf : 0][t][p] = (pa + pb) * 0.125f * 0x1p-26f;
+            } else {
+                bs[buf][i / SB][i % SB] = ss[k][0];
             }
+        }
+        if (WS == NTH || tid < WS) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const uint32_t x = sw[2 * q], y = sw[2 * q + 1];
+                const gm_h2 hx = __builtin_bit_cast(gm_h2, x), hy = __builtin_bit_cast(gm_h2, y);
+                *(gm_f4*)&bw[buf][wb][8 * wg + 4 * q] = (gm_f4){(float)hx[0], (float)hx[1], (float)hy[0], (float)hy[1]};
+            }
+        }
+    };
+
+    gm_f4 acc[TT];
+#pragma unroll
+    for (int t = 0; t < TT; t++) acc[t] = (gm_f4){0.0f, 0.0f, 0.0f, 0.0f};
+
+    // LDS operands of G blocks, read one set ahead of their MFMAs; the token
+    // scales (and xm_s) of a quad are read with its first set
+    long bf[2][G][TT];
+    float wsr[2][G][4];
+    gm_i4 c0 = {(int)BASE, (int)BASE, (int)BASE, (int)BASE};
+    asm("" : "+v"(c0));  // loop-invariant registers
+    float xs[2][TT][4];
+    float xm[2][TT][2];
+    auto lds_set = [&](int buf, int b, int slot, int xslot) {
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            const gm_f4 y = *(const gm_f4*)&bw[buf][b + g][16 * w + 4 * kc];
+#pragma unroll
+            for (int v = 0; v < 4; v++) wsr[slot][g][v] = y[v];
+#pragma unroll
+            for (int t = 0; t < TT; t++) bf[slot][g][t] = *(const long*)&bq[buf][b + g][32 * (16 * t + i16) + 8 * kc];
+        }
+        if (b % 4 == 0) {
 #pragma unroll
             for (int t = 0; t < TT; t++) {
-                const gm_h8 bf = bfr[sb & 1][t];
+                const gm_f4 x = *(const gm_f4*)&bs[buf][16 * t + i16][b];
 #pragma unroll
-                for (int f = 0; f < RF; f++) {
-                    // float(ws) * xs as one mixed-precision FMA with a +0
-                    // addend: the same rounding as the product, and a zero
-                    // product's sign cannot reach acc, which is never -0.
-                    // All four before their uses, so no product is read by
-                    // the instruction right after the one writing it.
-                    float wx[4];
-#pragma unroll
-                    for (int v = 0; v < 4; v++) wx[v] = __builtin_fmaf((float)wsh[f][v], xs[t], 0.0f);
-                    const gm_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[f], bf, (gm_f4){0.0f, 0.0f, 0.0f, 0.0f},
-                                                                         0, 0, 0);
-#pragma unroll
-                    for (int v = 0; v < 4; v++) acc[f][t][v] = fmaf(d[v], wx[v], acc[f][t][v]);
+                for (int j = 0; j < 4; j++) xs[xslot][t][j] = x[j];
+                if (ASYM) {
+                    const float* y = &bm[ASYM ? buf : 0][16 * t + i16][b / 2];
+                    xm[xslot][t][0] = y[0];
+                    xm[xslot][t][1] = y[1];
                 }
             }
         }
     };
+    gm_f4 dk[TT];   // modes 13 / 14: the even block's dots and the pair's d,
+    float dsk[4];   // held across the odd block
+    // one quad: nibbles of ring slot s, blocks b .. b + 3 of stage buffer buf
+    // (nb of them in range), the next quad's first set from LDS when there is
+    // one in the stage
+    auto quad = [&](int s, int buf, int b, int nb, int x, bool more) {
+        uint32_t t0 = wn[s][0], t1 = wn[s][1], t2 = wn[s][2], t3 = wn[s][3];
+        skp_transpose(t0, t1, t2, t3);
+        const uint32_t tw[4] = {t0, t1, t2, t3};
+        uint32_t th[4] = {0u, 0u, 0u, 0u};
+        if (MODE == 14) {
+            th[0] = wh[s][0];
+            th[1] = th[0] >> 4;
+            th[2] = wh[s][1];
+            th[3] = th[2] >> 4;
+            skp_transpose(th[0], th[1], th[2], th[3]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int slot = G == 4 ? x : (j / G) & 1, g = j % G;
+            if (g == 0) {
+                // the set after this one
+                if (j + G < 4)
+                    lds_set(buf, b + j + G, slot ^ 1, x);
+                else if (more)
+                    lds_set(buf, b + 4, slot ^ 1, x ^ 1);
+            }
+            if (j >= nb) break;  // uniform
+            uint32_t lo, hi;
+            if (!ASYM) {
+                // 16 (u - 8) as int8: the nibble with its top bit flipped, in
+                // the byte's upper half
+                lo = ((tw[j] << 4) ^ 0x80808080u) & 0xF0F0F0F0u;
+                hi = (tw[j] ^ 0x80808080u) & 0xF0F0F0F0u;
+            } else {
+                lo = tw[j] & 0x0F0F0F0Fu;
+                hi = (tw[j] >> 4) & 0x0F0F0F0Fu;
+                if (MODE == 14) {
+                    lo |= (th[j] << 4) & 0x30303030u;
+                    hi |= (th[j] << 2) & 0x30303030u;
+                }
+            }
+            const long a = (long)(((uint64_t)hi << 32) | lo);
+            const float(&ws)[4] = wsr[slot][g];
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                const gm_i4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bf[slot][g][t], c0, 0, 0, 0);
+                const float sx = xs[x][t][j];
+                float d[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int di_v = di[v];
+                    d[v] = __builtin_bit_cast(float, di_v) - __builtin_bit_cast(float, BASE);
+                }
+                if (!ASYM) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float p = ws[v] * sx;
+                        acc[t][v] = fmaf(d[v], p, acc[t][v]);
+                    }
+                } else if ((j & 1) == 0) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) dk[t][v] = d[v];
+                } else {
+                    const float sx0 = xs[x][t][j - 1], sm_ = xm[x][t][j >> 1];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float p1 = d[v] * sx;
+                        const float fd = fmaf(dk[t][v], sx0, p1);
+                        acc[t][v] = fmaf(fd, dsk[v], acc[t][v]);
+                        acc[t][v] = fmaf(ws[v], sm_, acc[t][v]);
+                    }
+                }
+            }
+            if (ASYM && (j & 1) == 0) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) dsk[v] = ws[v];
+            }
+        }
+    };
 
-    // prologue: stage 0 into LDS buffer 0, weights of stage 0
     stage_load(0);
-    weights_load(0, wn[0], wh[0]);
+#pragma unroll
+    for (int q = 0; q < PF; q++) wload(q, q);
     stage_store(0);
     __syncthreads();
-    int st = 0;
-    for (; st + 2 <= n_st; st += 2) {
-        stage_load(st + 1);
-        weights_load(st + 1, wn[1], wh[1]);
-        compute(st, 0, wn[0], wh[0]);
-        stage_store(1);
-        __syncthreads();
-        // on the last pair this stages clamped data that is never computed;
-        // the loop body has no branch around its loads
-        stage_load(st + 2);
-        weights_load(st + 2, wn[0], wh[0]);
-        compute(st + 1, 1, wn[1], wh[1]);
-        stage_store(0);
-        __syncthreads();
+    for (int st0 = 0; st0 < n_st; st0 += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int st = st0 + h;
+            if (st >= n_st) break;  // uniform
+            stage_load(st + 1);
+            lds_set(h, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < QS; i++) {
+                const int b = st * SB + 4 * i, s = (h * QS + i) % PF;
+                if (b < n_blk) quad(s, h, 4 * i, n_blk - b, i & 1, i + 1 < QS);
+                wload(st * QS + i + PF, s);
+            }
+            if (st + 1 < n_st) stage_store(h ^ 1);
+            __syncthreads();
+        }
     }
-    if (st < n_st) compute(st, 0, wn[0], wh[0]);
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[t][v] *= ASYM ? 0x1p26f : 0x1p22f;
 
     if constexpr (SWI) {
         // SwiGLU + prep of the down input for the workgroup's 64 columns
         // (one 64-block, blk) of the M tokens m0 .. m0 + 63.  Lane l of wave
-        // w holds acc[0][t][v] for column c = 16 (w & 3) + 4 (l / 16) + v and
+        // w holds acc[t][v] for column c = 16 (w & 3) + 4 (l / 16) + v and
         // token 16 t + l % 16; x[w & 3][t][v][l] in the LDS of the stage
         // buffers (free once every wave is past its last block) exchanges
         // them: the up waves write theirs, the gate waves replace them by
         // swiglu1(gate, up) (swiglu_prep_lane's arithmetic), then each 16-lane
         // row preps one token's block as swiglu_prep_lane does.
-        float* x = (float*)&bq[0][0][0][0];
+        float* x = (float*)&bq[0][0][0];
         static_assert(sizeof(bq) >= 4 * TT * 4 * 64 * sizeof(float), "the exchange fits the stage buffers");
         auto xi = [&](int ww, int t, int v, int ln) { return ((ww * TT + t) * 4 + v) * 64 + ln; };
         const int blk = (gb * 8) >> 6;  // gb: the wave's first group; a block is 8 groups
         __syncthreads();
-        if (wu >= 4) {
+        if (w >= 4) {
 #pragma unroll
             for (int t = 0; t < TT; t++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) x[xi(wl, t, v, l)] = acc[0][t][v];
+                for (int v = 0; v < 4; v++) x[xi(wl, t, v, l)] = acc[t][v];
         }
         __syncthreads();
-        if (wu < 4) {
+        if (w < 4) {
             const uint8_t* sg = A.swsign ? A.swsign + 8 * blk : nullptr;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int c = 16 * wl + 4 * kc + v;
                 const uint32_t neg = sg ? (sg[c >> 3] >> (c & 7)) & 1u : 0u;
 #pragma unroll
-                for (int t = 0; t < TT; t++) x[xi(wl, t, v, l)] = swiglu1(acc[0][t][v], x[xi(wl, t, v, l)], A.swdz, neg);
+                for (int t = 0; t < TT; t++) x[xi(wl, t, v, l)] = swiglu1(acc[t][v], x[xi(wl, t, v, l)], A.swdz, neg);
             }
         }
         __syncthreads();
         const int R = tid >> 4, r = tid & 15, I = A.swI, nbI = I >> 5;
 #pragma unroll
-        for (int pass = 0; pass < NT / 32; pass++) {
+        for (int pass = 0; pass < (NT + 31) / 32; pass++) {
             const int tok = R + 32 * pass, mt = m0 + tok;
-            if (mt < M) {  // uniform over the 16-lane row
+            if (tok < NT && mt < M) {  // uniform over the 16-lane row
                 float v4[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
@@ -505,20 +493,365 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MODE ==
         }
         return;
     }
-    // rows 16 RF w + 16f + 4kc + v of the workgroup, token m0 + 16t + i16
+    // rows 16 w + 4kc + v of the workgroup, token m0 + 16t + i16
+    const int grp = gb + 2 * w + (kc >> 1);
+    if (grp >= J.g1) return;
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+        const int m = m0 + 16 * t + i16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int r = grp * 8 + (kc & 1) * 4 + v;
+            if (r < J.rows) J.out[(size_t)m * J.ldo + r] = acc[t][v];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k_gemm_x32: 32 x 32 tiles, for launches with tiles enough to fill the chip.
+// A 32x32x32 MFMA costs 8.2 cycles per 16 x 16 outputs where a 16x16x32 one
+// costs 17, and a fragment read from LDS feeds twice the outputs.  The tokens
+// are the MFMA's A and the weights its B, so a lane holds one weight row: one
+// weight scale per lane and block, and stores of 32 consecutive rows.
+//
+// Workgroup of 4 waves = 2 row waves x 2 token waves: 64 RF weight rows x 64
+// tokens; a wave holds RF 32-row fragments x 32 tokens.  SWI: fragment 0 is
+// 32 rows of gate and fragment 1 the same rows of up, so the SwiGLU needs no
+// exchange and the workgroup's 64 columns are one 64-block of the down input.
+template <int RF, int MODE, bool SWI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && MODE == 12 ? 3 : 2))) void k_gemm_x32(GmArgs A) {
+    constexpr int NT = 64, SB = 8;           // tokens per workgroup, blocks per LDS stage
+    constexpr int PS = SB / 2;               // block pairs per stage
+    constexpr int GPW = 8 * RF;              // 8-row groups per workgroup
+    constexpr bool ASYM = MODE != 12;
+    constexpr uint32_t BASE = 0x3e22f983u;   // 1 / (2 pi), an inline constant
+    static_assert(!SWI || (RF == 2 && MODE == 12), "fragment 0 gate, fragment 1 up");
+    __shared__ __align__(16) uint8_t aq[2][SB][NT * 32 + 32];  // int8 activations [stage][block][token][k]
+    __shared__ __align__(16) float xl[2][SB][NT + 8];        // token scales
+    __shared__ __align__(16) float ml[ASYM ? 2 : 1][SB / 2][NT + 8];  // xm_s of the 64-blocks (modes 13 / 14)
+    __shared__ __align__(16) float wl[2][SB][GPW * 8 + 8];   // weight scales
+    const int jx = blockIdx.x >> 3, ty = jx % A.gy;
+    const int rt = (jx / A.gy) * 8 + (blockIdx.x & 7);
+    if (rt >= A.tb[A.n_jobs]) {
+        const int zi = rt - A.tb[A.n_jobs];
+        if (zi < A.zt) {
+            const int r = A.z0 + 64 * zi + (threadIdx.x & 63);
+            for (int t = threadIdx.x >> 6; t < NT; t += 4) {
+                const int m = ty * NT + t;
+                if (m < A.M && r < A.z1) A.zo[(size_t)m * A.zld + r] = 0.0f;
+            }
+        }
+        return;
+    }
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, r32 = l & 31, h = l >> 5;
+    const int wr = w & 1, wt = w >> 1;
+    int ji = 0;
+    if (!SWI) {
+        if (A.n_jobs > 1 && rt >= A.tb[1]) ji = 1;
+        if (A.n_jobs > 2 && rt >= A.tb[2]) ji = 2;
+    }
+    const GmJob& J = ji == 0 ? A.j[0] : ji == 1 ? A.j[1] : A.j[2];
+    const int8_t* const Jq = ji == 0 ? A.j[0].q : ji == 1 ? A.j[1].q : A.j[2].q;
+    const float* const Js = ji == 0 ? A.j[0].s : ji == 1 ? A.j[1].s : A.j[2].s;
+    const int32_t* const Jm = ji == 0 ? A.j[0].m : ji == 1 ? A.j[1].m : A.j[2].m;
+    const int gb = SWI ? rt * 8 : J.g0 + (rt - A.tb[ji]) * GPW;  // first group of the workgroup
+    const int m0 = ty * NT;
+    const int K = A.K, M = A.M, n_blk = K >> 5, n_st = (n_blk + SB - 1) / SB;
+    const size_t gstride = (size_t)n_blk * (MODE == 14 ? 208 : 144);
+    const auto rsrc = [](const void* p, size_t n) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(n < 0xFFFFFFFFu ? n : 0xFFFFFFFFu), GM_RSRC3);
+    };
+    // a fragment's first group (fragment f: rows 32 (RF wr + f) of the
+    // workgroup; SWI: rows 32 wr of job f), its descriptor and lane offset
+    __amdgpu_buffer_rsrc_t rw[RF];
+    uint32_t on[RF], oh[RF];
 #pragma unroll
     for (int f = 0; f < RF; f++) {
-        const int grp = gb + 2 * RF * w + 2 * f + (kc >> 1);
-        if (grp >= J.g1) continue;
+        const GmJob& Jf = SWI ? A.j[f] : J;
+        const int gf = min(gb + (SWI ? 4 * wr : 4 * (RF * wr + f)), Jf.g1 - 1);
+        rw[f] = rsrc(Jf.g + (size_t)gf * gstride, (size_t)(Jf.g1 - gf) * gstride);
+        const int ga = min(gb + (SWI ? 4 * wr : 4 * (RF * wr + f)) + (r32 >> 3), Jf.g1 - 1);
+        on[f] = (uint32_t)((size_t)(ga - gf) * gstride + (size_t)n_blk * 16 + (r32 & 7) * 16 + h * 128);
+        oh[f] = (uint32_t)((size_t)(ga - gf) * gstride + (size_t)n_blk * 144 + (r32 & 7) * 8 + h * 64);
+    }
+    constexpr int PF = ASYM && RF == 2 ? 2 : 4;  // block pairs of nibbles in flight
+    static_assert((2 * PS) % PF == 0, "ring slots are static over two stages");
+    gm_u4 wn[PF][RF];
+    gm_u2 wh[PF][RF];
+    auto wload = [&](int p, int slot) {
 #pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const int m = m0 + 16 * t + i16;
-            if (m >= M) continue;
+        for (int f = 0; f < RF; f++) {
+            wn[slot][f] = __builtin_bit_cast(
+                gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rw[f], on[f] + (uint32_t)p * 256u, 0, 0));
+            if (MODE == 14)
+                wh[slot][f] = __builtin_bit_cast(
+                    gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rw[f], oh[f] + (uint32_t)p * 128u, 0, 0));
+        }
+    };
+    // staging: 16-byte piece c = tid + 256 k of a token's SB 32 contiguous
+    // bytes; scale i: token i / SB, block i % SB (modes 13 / 14: token, pair)
+    constexpr int CPT = NT * SB * 2 / 256, SPT = NT * SB / 256;  // 4, 2
+    gm_u4 sq[CPT];
+    float ss[SPT];
+    int32_t sm[2];
+    gm_u4 sw;
+    const __amdgpu_buffer_rsrc_t rq = rsrc(Jq, (size_t)M * K);
+    const __amdgpu_buffer_rsrc_t rs = rsrc(Js, (size_t)M * n_blk * 4);
+    const __amdgpu_buffer_rsrc_t rm = rsrc(ASYM ? (const void*)Jm : (const void*)Js, (size_t)M * n_blk * 4);
+    // weight scales: thread t < 8 GPW stages the 16 bytes of group t / SB,
+    // block t % SB (SWI: groups 8 .. 15 are job 1's, threads 64 .. 127)
+    constexpr int WS = GPW * SB;
+    const int wg = (tid % WS) / SB, wb = tid % SB;
+    const GmJob& JG = SWI ? (w & 1 ? A.j[1] : A.j[0]) : J;
+    const __amdgpu_buffer_rsrc_t rg = rsrc(JG.g + (size_t)gb * gstride, (size_t)(JG.g1 - gb) * gstride);
+    const uint32_t og = (uint32_t)((size_t)(min(gb + (SWI ? (wg & 7) : wg), JG.g1 - 1) - gb) * gstride + wb * 16);
+    uint32_t qo[CPT], so[SPT];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = grp * 8 + (kc & 1) * 4 + v;
-                if (r < J.rows) J.out[(size_t)m * J.ldo + r] = acc[f][t][v];
+    for (int k = 0; k < CPT; k++) {
+        const int c = tid + 256 * k;
+        qo[k] = (uint32_t)(min(m0 + c / (2 * SB), M - 1) * K + 16 * (c % (2 * SB)));
+    }
+#pragma unroll
+    for (int k = 0; k < SPT; k++) {
+        const int i = tid + 256 * k;
+        so[k] = ASYM ? (uint32_t)(4 * (min(m0 + tid / PS, M - 1) * n_blk + 2 * (tid % PS)))
+                     : (uint32_t)(4 * (min(m0 + i / SB, M - 1) * n_blk + i % SB));
+    }
+    auto stage_load = [&](int st) {
+#pragma unroll
+        for (int k = 0; k < CPT; k++)
+            sq[k] = __builtin_bit_cast(gm_u4,
+                                       __builtin_amdgcn_raw_buffer_load_b128(rq, qo[k] + (uint32_t)st * (SB * 32u), 0, 0));
+        if (ASYM) {
+            const uint32_t o = so[0] + (uint32_t)st * (SB * 4u);
+            const gm_u2 a = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
+            const gm_u2 b = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rm, o, 0, 0));
+            const uint32_t a0 = a[0], a1 = a[1];
+            ss[0] = __builtin_bit_cast(float, a0);
+            ss[1] = __builtin_bit_cast(float, a1);
+            sm[0] = (int32_t)b[0];
+            sm[1] = (int32_t)b[1];
+        } else {
+#pragma unroll
+            for (int k = 0; k < SPT; k++) {
+                const uint32_t a = __builtin_amdgcn_raw_buffer_load_b32(rs, so[k] + (uint32_t)st * (SB * 4u), 0, 0);
+                ss[k] = __builtin_bit_cast(float, a);
             }
+        }
+        sw = __builtin_bit_cast(gm_u4, __builtin_amdgcn_raw_buffer_load_b128(rg, og + (uint32_t)st * (SB * 16u), 0, 0));
+    };
+    auto stage_store = [&](int buf) {
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            const int c = tid + 256 * k;
+            *(gm_u4*)&aq[buf][(c >> 1) % SB][32 * (c / (2 * SB)) + 16 * (c & 1)] = sq[k];
+        }
+        if (ASYM) {
+            const int t = tid / PS, p = tid % PS;
+            xl[buf][2 * p][t] = ss[0];
+            xl[buf][2 * p + 1][t] = ss[1];
+            const float pa = (float)sm[0] * ss[0], pb = (float)sm[1] * ss[1];
+            ml[ASYM ? buf : 0][p][t] = (pa + pb) * 0.125f * 0x1p-26f;
+        } else {
+#pragma unroll
+            for (int k = 0; k < SPT; k++) {
+                const int i = tid + 256 * k;
+                xl[buf][i % SB][i / SB] = ss[k];
+            }
+        }
+        if (tid < WS) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const uint32_t a = sw[2 * q], b = sw[2 * q + 1];
+                const gm_h2 x = __builtin_bit_cast(gm_h2, a), y = __builtin_bit_cast(gm_h2, b);
+                *(gm_f4*)&wl[buf][wb][wg * 8 + 4 * q] = (gm_f4){(float)x[0], (float)x[1], (float)y[0], (float)y[1]};
+            }
+        }
+    };
+
+    float acc[RF][16];
+#pragma unroll
+    for (int f = 0; f < RF; f++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[f][v] = 0.0f;
+    const bool live = m0 + 32 * wt < M;  // uniform: the wave has a token to compute
+
+    // LDS operands of one block
+    gm_i4 af[2];
+    float xs[2][16];
+    float ws[2][RF];
+    auto lds_blk = [&](int buf, int b, int slot) {
+        af[slot] = *(const gm_i4*)&aq[buf][b][32 * (32 * wt + r32) + 16 * h];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const gm_f4 x = *(const gm_f4*)&xl[buf][b][32 * wt + 8 * g + 4 * h];
+#pragma unroll
+            for (int v = 0; v < 4; v++) xs[slot][4 * g + v] = x[v];
+        }
+#pragma unroll
+        for (int f = 0; f < RF; f++) ws[slot][f] = wl[buf][b][(SWI ? 64 * f + 32 * wr : 32 * (RF * wr + f)) + r32];
+    };
+    float dk[RF][16];  // modes 13 / 14: the even block's dots, d and token scales
+    float dd[RF];
+    float xk[16];
+    gm_i16 c0;  // loop-invariant, so that the MFMAs share one set of registers
+#pragma unroll
+    for (int v = 0; v < 16; v++) c0[v] = (int)BASE;
+    asm("" : "+v"(c0));
+    // block pair p of a stage (blocks 2 p, 2 p + 1; nb of them in range)
+    auto pair = [&](int s, int buf, int p, int nb, bool more) {
+        gm_i4 wa[2][RF];
+#pragma unroll
+        for (int f = 0; f < RF; f++) {
+            uint32_t w0 = wn[s][f][0], w1 = wn[s][f][1], w2 = wn[s][f][2], w3 = wn[s][f][3];
+            // chunks 2 h, 2 h + 1 of both blocks
+            const auto e0 = __builtin_amdgcn_permlane32_swap(w0, w2, false, false);
+            const auto e1 = __builtin_amdgcn_permlane32_swap(w1, w3, false, false);
+            const uint32_t c[2][2] = {{e0[0], e1[0]}, {e0[1], e1[1]}};
+            uint32_t hb[2] = {0u, 0u};
+            if (MODE == 14) {
+                // the block's high-bit word h (chunks 2 h: low nibbles, 2 h + 1: high)
+                const auto eh = __builtin_amdgcn_permlane32_swap(wh[s][f][0], wh[s][f][1], false, false);
+                hb[0] = eh[0];
+                hb[1] = eh[1];
+            }
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    uint32_t lo, hi;
+                    if (!ASYM) {
+                        lo = ((c[b][q] << 4) ^ 0x80808080u) & 0xF0F0F0F0u;
+                        hi = (c[b][q] ^ 0x80808080u) & 0xF0F0F0F0u;
+                    } else {
+                        lo = c[b][q] & 0x0F0F0F0Fu;
+                        hi = (c[b][q] >> 4) & 0x0F0F0F0Fu;
+                        if (MODE == 14) {
+                            lo |= (q ? hb[b] : hb[b] << 4) & 0x30303030u;
+                            hi |= (q ? hb[b] >> 2 : hb[b] << 2) & 0x30303030u;
+                        }
+                    }
+                    wa[b][f][2 * q] = (int)lo;
+                    wa[b][f][2 * q + 1] = (int)hi;
+                }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if (b == 0 || more) lds_blk(buf, 2 * p + b + 1, b ^ 1);
+            if (b >= nb) break;  // uniform
+            gm_i16 d[RF];
+#pragma unroll
+            for (int f = 0; f < RF; f++) {
+                d[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b], wa[b][f], c0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int f = 0; f < RF; f++) {
+                if (!ASYM) {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const int di = d[f][v];
+                        const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        const float pr = xs[b][v] * ws[b][f];
+                        acc[f][v] = fmaf(x, pr, acc[f][v]);
+                    }
+                } else if (b == 0) {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const int di = d[f][v];
+                        dk[f][v] = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        xk[v] = xs[0][v];
+                    }
+                    dd[f] = ws[0][f];
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const int di = d[f][v];
+                        const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        const float p1 = x * xs[1][v];
+                        const float fd = fmaf(dk[f][v], xk[v], p1);
+                        acc[f][v] = fmaf(fd, dd[f], acc[f][v]);
+                    }
+                }
+            }
+            if (ASYM && b == 1) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const gm_f4 y = *(const gm_f4*)&ml[ASYM ? buf : 0][p][32 * wt + 8 * g + 4 * h];
+#pragma unroll
+                    for (int f = 0; f < RF; f++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) acc[f][4 * g + v] = fmaf(ws[1][f], y[v], acc[f][4 * g + v]);
+                }
+            }
+        }
+    };
+
+    stage_load(0);
+#pragma unroll
+    for (int p = 0; p < PF; p++) wload(p, p);
+    stage_store(0);
+    __syncthreads();
+    for (int st0 = 0; st0 < n_st; st0 += 2) {
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            const int st = st0 + hh;
+            if (st >= n_st) break;  // uniform
+            stage_load(st + 1);
+            if (live) {
+                lds_blk(hh, 0, 0);
+#pragma unroll
+                for (int i = 0; i < PS; i++) {
+                    const int b = st * SB + 2 * i, s = (hh * PS + i) % PF;
+                    if (b < n_blk) pair(s, hh, i, n_blk - b, i + 1 < PS);
+                    wload(st * PS + i + PF, s);
+                }
+            }
+            if (st + 1 < n_st) stage_store(hh ^ 1);
+            __syncthreads();
+        }
+    }
+    const float rescale = ASYM ? 0x1p26f : 0x1p22f;
+#pragma unroll
+    for (int f = 0; f < RF; f++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[f][v] *= rescale;
+
+    if constexpr (SWI) {
+        constexpr int XS = 68;
+        float* x = (float*)&aq[0][0][0];  // [token][column], rows padded
+        static_assert(sizeof(aq) >= NT * XS * sizeof(float), "the exchange fits the stage buffers");
+        const int col = 32 * wr + r32;
+        const uint32_t neg = A.swsign ? (A.swsign[8 * rt + (col >> 3)] >> (col & 7)) & 1u : 0u;
+        if (live) {
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                x[(32 * wt + 8 * (v >> 2) + 4 * h + (v & 3)) * XS + col] = swiglu1(acc[0][v], acc[1][v], A.swdz, neg);
+        }
+        __syncthreads();
+        const int R = tid >> 4, r = tid & 15, I = A.swI, nbI = I >> 5;
+#pragma unroll
+        for (int pass = 0; pass < NT / 16; pass++) {
+            const int tok = R + 16 * pass, mt = m0 + tok;
+            if (mt < M) {  // uniform over the 16-lane row
+                float v4[4];
+                const gm_f4 y = *(const gm_f4*)&x[tok * XS + 4 * r];
+#pragma unroll
+                for (int k = 0; k < 4; k++) v4[k] = y[k];
+                row_prep64(v4, r, rt, A.swo.q + (size_t)mt * I, A.swo.s + (size_t)mt * nbI, A.swo.m + (size_t)mt * nbI,
+                           A.swo.h ? A.swo.h + (size_t)mt * I : nullptr);
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int f = 0; f < RF; f++) {
+        const int row = (gb + 4 * (RF * wr + f)) * 8 + r32;
+        if (row >= J.g1 * 8 || row >= J.rows) continue;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int m = m0 + 32 * wt + 8 * (v >> 2) + 4 * h + (v & 3);
+            if (m < M) J.out[(size_t)m * J.ldo + row] = acc[f][v];
         }
     }
 }
@@ -1110,22 +1443,30 @@ static GmKernel gm_skp_of(int nr) {
 }
 }
 
+extern "C++" {
+template <int MODE>
+static GmKernel gm_of(bool x32, int rf, int tt) {
+    if (!x32) return tt == 1 ? k_gemm_mfma<1, MODE, 4, false> : k_gemm_mfma<2, MODE, 4, false>;
+    if constexpr (MODE != 14)
+        if (rf == 2) return k_gemm_x32<2, MODE, false>;
+    return k_gemm_x32<1, MODE, false>;
+}
+}
+
 // Gate and up of M > 16 tokens with the SwiGLU + dead zone + prep of the down
-// input in the same launch (k_gemm_mfma<..., true>): a workgroup's
-// waves 0-3 compute 64 rows of gate, waves 4-7 the same 64 rows of up, from
-// the activations both share, and the workgroup preps those 64 columns of
-// every token into out.  -1 (nothing launched) when the shapes do not allow
-// it: mode 12, one shared input, every row of equal gate / up matrices with
-// 64 | rows, fp16 activations, and out distinct from the input.  Unlike the
-// plain gate+up launch it pays at every M > 16 (pp32 8.7 -> 8.6 ms, pp64 9.3
-// -> 9.1, pp128 10.2 either way, pp512 20.7 -> 19.8 at the 8B shape).
+// input in the same launch: the workgroup that computes 64 rows of gate and
+// the same of up preps those 64 columns of its tokens into out.  -1 (nothing
+// launched) when the shapes do not allow it: mode 12, one shared input, every
+// row of equal gate / up matrices with 64 | rows, and out distinct from the
+// input.  It pays at every M > 16: the fp32 gate and up rows are never written
+// and a launch goes (pp512 20.7 -> 19.8 ms when it was introduced).
 int32_t dpuf_hip_gemm_swiglu(void* s, int32_t M, const DpufGemvJob* jobs, float dz, const uint8_t* sign,
                              DpufPrep out) {
     const DpufGemvJob& a = jobs[0];
     const DpufGemvJob& b = jobs[1];
     const int I = a.w.rows;
     if (M <= 16 || a.w.mode != 12 || b.w.mode != 12 || a.w.cols != b.w.cols || b.w.rows != I || I % 64 ||
-        2 * I < GM_NW8_ROWS || a.g0 != 0 || b.g0 != 0 || a.g1 != I / 8 || b.g1 != I / 8 || !a.p.h || a.p.h != b.p.h ||
+        2 * I < GM_SWI_ROWS || a.g0 != 0 || b.g0 != 0 || a.g1 != I / 8 || b.g1 != I / 8 || !a.p.q || a.p.q != b.p.q ||
         a.p.s != b.p.s || !out.q || !out.s || !out.m || !out.h || out.h == a.p.h || out.q == a.p.q)
         return -1;
     if ((long long)M * a.w.cols >= (1ll << 30) || (long long)M * I >= (1ll << 30)) return -1;
@@ -1140,6 +1481,7 @@ int32_t dpuf_hip_gemm_swiglu(void* s, int32_t M, const DpufGemvJob* jobs, float 
         G.j[i].g1 = jobs[i].g1;
         G.j[i].rows = jobs[i].w.rows;
         G.j[i].h = jobs[i].p.h;
+            G.j[i].q = jobs[i].p.q;
         G.j[i].s = jobs[i].p.s;
         G.j[i].m = jobs[i].p.m;
         G.j[i].out = jobs[i].out;
@@ -1154,9 +1496,13 @@ int32_t dpuf_hip_gemm_swiglu(void* s, int32_t M, const DpufGemvJob* jobs, float 
     G.swdz = dz;
     G.swI = I;
     const int gx = (tiles + 7) & ~7;
-    G.gy = (M + 16 * GM_TT - 1) / (16 * GM_TT);
-    const dim3 grid = GM_XCD ? dim3(gx * G.gy) : dim3(gx, G.gy);
-    hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 12, 8, true>), grid, dim3(512), 0, ST(s), G);
+    // up to 32 tokens two 16-token tiles, else 32 x 32 tiles (M = 29: 32 us against
+    // 50, whose second token wave has nothing to do; M = 512: 204 against 178)
+    const bool x32 = M > 32;
+    const int nt = x32 ? 64 : 32;
+    G.gy = (M + nt - 1) / nt;
+    GmKernel k = x32 ? k_gemm_x32<2, 12, true> : k_gemm_mfma<2, 12, 8, true>;
+    hipLaunchKernelGGL(k, dim3(gx * G.gy), dim3(x32 ? 256 : 512), 0, ST(s), G);
     LAUNCHED("k_gemm_mfma");
     return 0;
 }
@@ -1167,22 +1513,17 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
     {
         GmArgs G;
         memset(&G, 0, sizeof G);
-        int t = 0;
-        // 8-wave workgroups (128 rows sharing one staged token tile) for the
-        // launches with the most rows, 4-wave ones otherwise
-        int rows_all = 0;
-        for (int i = 0; i < n_jobs; i++) rows_all += jobs[i].g1 > jobs[i].g0 ? 8 * (jobs[i].g1 - jobs[i].g0) : 0;
-        const int nw = jobs[0].w.mode == 12 && M > GM_NW8_MINM && rows_all >= GM_NW8_ROWS ? 8 : 4;
-        const int gpw = 2 * GM_RF * nw;
         G.n_jobs = n_jobs;
         G.K = jobs[0].w.cols;
         G.M = M;
+        int any = 0;
         for (int i = 0; i < n_jobs; i++) {
             G.j[i].g = jobs[i].w.g;
             G.j[i].g0 = jobs[i].g0;
             G.j[i].g1 = jobs[i].g1;
             G.j[i].rows = jobs[i].w.rows;
             G.j[i].h = jobs[i].p.h;
+            G.j[i].q = jobs[i].p.q;
             if ((long long)M * G.K >= (1ll << 30)) {
                 note(hipErrorInvalidValue, "dpuf_hip_gemv: M * K must stay below 2^30");
                 return;
@@ -1195,11 +1536,8 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
             G.j[i].m = jobs[i].p.m;
             G.j[i].out = jobs[i].out;
             G.j[i].ldo = jobs[i].ldo;
-            G.tb[i] = t;
-            const int ng = jobs[i].g1 - jobs[i].g0;
-            t += ng > 0 ? (ng + gpw - 1) / gpw : 0;
+            any += jobs[i].g1 > jobs[i].g0;
         }
-        G.tb[n_jobs] = t;
         if (zo && z1 > z0) {
             G.zo = zo;
             G.zld = zld;
@@ -1207,7 +1545,7 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
             G.z1 = z1;
             G.zt = (z1 - z0 + 63) / 64;
         }
-        if (t + G.zt <= 0) return;
+        if (any + G.zt <= 0) return;
         const int n_blk = G.K >> 5;
         const int mode = jobs[0].w.mode;  // one mode per launch (dpuf_hip_gemv groups them)
         long long gmax = 0;
@@ -1258,18 +1596,37 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
             LAUNCHED("k_gemm_sk");
             return;
         }
+        // The tile by the number of 16 x 16 tiles per SIMD (each a serial
+        // chain over K).  Measured, us (16 x 16 | 16 x 32 | 32 x 32 | 64 x 32
+        // per wave), mode 12: 4 096 rows, K = 12 288: 2 per SIMD 43 | 61 | 88 |
+        // 126; 4 per SIMD 86 | 81 | 90 | 126; 8 per SIMD 179 | 160 | 119 | 136.
+        // 6 144 rows, K = 4 096: 3 per SIMD 26 | 29 | 32 | 46; 6 per SIMD 46 |
+        // 39 | 37 | 47.  24 576 rows: 12 per SIMD 86 | 72 | 52 | 62; 48 per SIMD
+        // 312 | 254 | 200 | 190.  In mode 13 the wider wave is ahead sooner
+        // (24 576 rows, 9 per SIMD: 65 | 71 | 64; 6 per SIMD 42 | 43 | 53); in
+        // mode 14 its registers do not fit.
+        const int tm = (M + 15) / 16, simds = 4 * dpuf_hip_cu_count();
+        long long tiles = 0;
+        for (int i = 0; i < n_jobs; i++) {
+            const int ng = jobs[i].g1 - jobs[i].g0;
+            tiles += ng > 0 ? (long long)((ng + 1) / 2) * tm : 0;
+        }
+        const bool x32 = tiles >= 6ll * simds;
+        const int rf = x32 && mode != 14 && tiles >= (mode == 13 ? 8ll : 32ll) * simds ? 2 : 1;
+        const int tt = tiles >= 4ll * simds ? 2 : 1;
+        const int nt = x32 ? 64 : 16 * tt, gpw = 8 * rf;
+        int t = 0;
+        for (int i = 0; i < n_jobs; i++) {
+            G.tb[i] = t;
+            const int ng = jobs[i].g1 - jobs[i].g0;
+            t += ng > 0 ? (ng + gpw - 1) / gpw : 0;
+        }
+        G.tb[n_jobs] = t;
         // a multiple of 8 row tiles keeps a row tile's token tiles on one XCD
         const int gx = (t + G.zt + 7) & ~7;
-        G.gy = (M + 16 * GM_TT - 1) / (16 * GM_TT);
-        const dim3 grid = GM_XCD ? dim3(gx * G.gy) : dim3(gx, G.gy);
-        if (mode == 13)
-            hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 13, 4>), grid, dim3(256), 0, ST(s), G);
-        else if (mode == 14)
-            hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 14, 4>), grid, dim3(256), 0, ST(s), G);
-        else if (nw == 8)
-            hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 12, 8>), grid, dim3(512), 0, ST(s), G);
-        else
-            hipLaunchKernelGGL((k_gemm_mfma<GM_TT, GM_RF, 12, 4>), grid, dim3(256), 0, ST(s), G);
+        G.gy = (M + nt - 1) / nt;
+        GmKernel k = mode == 13 ? gm_of<13>(x32, rf, tt) : mode == 14 ? gm_of<14>(x32, rf, tt) : gm_of<12>(x32, rf, tt);
+        hipLaunchKernelGGL(k, dim3(gx * G.gy), dim3(256), 0, ST(s), G);
         LAUNCHED("k_gemm_mfma");
     }
 }

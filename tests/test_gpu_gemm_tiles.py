@@ -1,0 +1,49 @@
+"""The tile shapes of the GEMM above 16 tokens (16 x 16, 16 x 32, 32 x 32 and
+64 x 32 outputs per wave, chosen by the tiles per SIMD) against the oracle, bit
+for bit, in every mode: sizes on each side of the rule, rows that end inside a
+fragment, tokens that end inside a tile or leave a wave of a workgroup without
+any, and K from one 64-block to several LDS stages with a partial last one."""
+import numpy as np
+import pytest
+
+from dpuf_amd import model as M
+from test_gpu_configs import bits_equal, log, maxdiff
+
+pytestmark = pytest.mark.gpu
+
+NAMES = {12: "hadamard4_packed", 13: "had4_asym", 14: "had6"}
+# (rows, tokens): tiles per SIMD of a 256-CU device in the comment
+SIZES = [
+    (40, 17),      # < 1
+    (4136, 40),    # < 1, the last fragment one group
+    (4136, 250),   # 4.05: 16 x 32
+    (5000, 270),   # 5.2: one token past a 16-token tile
+    (6152, 250),   # 6.02: 32 x 32
+    (8200, 289),   # 9.5: 64 x 32 in mode 13; a single token in the last workgroup
+    (33000, 257),  # 34: 64 x 32 in mode 12
+]
+
+
+@pytest.mark.parametrize("mode", [12, 13, 14])
+@pytest.mark.parametrize("cols", [64, 320, 1088])
+@pytest.mark.parametrize("rows,m", SIZES)
+def test_gemm_tiles(eng, orc, mode, cols, rows, m):
+    if rows * m * cols > 5e9:
+        cols = 192  # the oracle's time
+    W = M.random_normal(rows * cols, 0.02, 7 + mode, f"t{rows}x{cols}").reshape(rows, cols)
+    blob, d = M.pack_matrix(W, M.sign_bits(cols, 7, f"ts{rows}x{cols}"), mode=mode)
+    x = np.random.default_rng(rows + cols + m).standard_normal((m, cols)).astype(np.float32)
+    x[m - 1, :32] = 1e-6
+    out_g = np.full((m, rows), np.nan, np.float32)
+    out_o = np.full((m, rows), np.nan, np.float32)
+    log(f"mode {mode} rows={rows} cols={cols} M={m}")
+    getattr(eng, f"dpuf_matmul_qr_{NAMES[mode]}_f32")(m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base,
+                                                      d.tile_offsets, d.sign_bits, M.ptr(out_g))
+    if mode == 12:
+        orc.orc_matmul_f32(m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base, d.tile_offsets, d.sign_bits,
+                           M.ptr(out_o))
+    else:
+        orc.orc_matmul_asym_f32(int(mode == 14), m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base, d.tile_offsets,
+                                d.sign_bits, M.ptr(out_o))
+    assert np.isfinite(out_o).all()
+    assert bits_equal(out_g, out_o), maxdiff(out_g, out_o)
