@@ -942,6 +942,15 @@ int32_t dpuf_hip_attn_decode_rope(void* s, int32_t lmax, float* q, const float* 
                       warm);
 }
 
+int32_t dpuf_hip_attn_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v,
+                               const float* qn, const float* kn, float eps, const float* cos_tab, const float* sin_tab,
+                               float* const* kcs, float* const* vcs, size_t l_off, float* out, float* scores,
+                               const int32_t* pos, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq,
+                               float scale) {
+    return attn_wide_sessions(s, n, lmax, q, k, v, qn, kn, eps, cos_tab, sin_tab, kcs, vcs, l_off, out, scores, pos, n_q,
+                              n_kv, hd, max_seq, scale);
+}
+
 void dpuf_hip_attn(void* s, int32_t M, const float* q, const float* kc, const float* vc, float* out, float* scores,
                    const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq, float scale) {
     const int groups = n_q / n_kv;

@@ -39,18 +39,30 @@
 // distinct banks.
 
 
-template <int HD, int GM, bool ROPE>
+// MS: one token of each of gridDim.z sessions (ROPE only).
+template <int HD, int GM, bool ROPE, bool MS>
 __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, const float* __restrict__ kc,
                                                   const int32_t* __restrict__ pos0p, int n_q, int n_kv, int max_seq,
-                                                  float scale, float* __restrict__ S, ScRope ra) {
+                                                  float scale, float* __restrict__ S, ScRope ra, MsTab ms) {
+    static_assert(!MS || ROPE, "sessions take the RoPE in the launch");
     constexpr int LD = HD + 8, E = HD / 64;
     extern __shared__ __align__(16) float sm[];
     float* ks = sm;               // [AS_KC][LD]
     float* qs = ks + AS_KC * LD;  // [GM][HD]
     const int kvh = blockIdx.x, t0 = blockIdx.y * AS_KC, tid = threadIdx.x;
     const int G = n_q / n_kv;
-    const int pos = *pos0p, L = pos + 1;
+    const int z = MS ? blockIdx.z : 0;
+    const int pos = pos0p[z], L = pos + 1;
     if (t0 >= L) return;  // every key of the chunk is past the row
+    if (MS) {
+        q += (size_t)z * ms.q_ld;
+        ra.k += (size_t)z * ms.kv_ld;
+        ra.v += (size_t)z * ms.kv_ld;
+        ra.kc = ms.kcs[z] + ms.lo;
+        ra.vc = ms.vcs[z] + ms.lo;
+        kc = ra.kc;
+        S += (size_t)z * ms.sc_ld;
+    }
     // ROPE units of wave tid / 64: q rows u < GM, then (if this chunk holds
     // the position) the new K row as unit GM; a wave takes u = w, w + 4, w + 8
     const int w = tid >> 6, lane = tid & 63;
@@ -220,20 +232,21 @@ DEV void smx_warm(const SmxWarm& W, int L, int max_seq) {
     asm volatile("" ::"v"(acc));  // the loaded values count as used: the reads stay
 }
 
+// blockIdx.y: the session (score rows sc_ld apart).
 template <int SEG>
 __global__ __launch_bounds__(SMX_NT) void k_attn_smx(float* __restrict__ S, const int32_t* __restrict__ pos0p,
-                                                  int max_seq, SmxWarm W) {
+                                                  int max_seq, SmxWarm W, size_t sc_ld) {
     constexpr int LDT = 8 * SEG + 4;  // row stride of the transposed copy
     __shared__ __align__(16) float tr[8][LDT];
     __shared__ float tail[8];
     __shared__ float red[SMX_NT / 64];
     __shared__ float part[8];
-    const int L = *pos0p + 1, n8 = L & ~7;
+    const int L = pos0p[blockIdx.y] + 1, n8 = L & ~7;
     if ((int)blockIdx.x >= W.n_rows) {
         smx_warm(W, L, max_seq);
         return;
     }
-    float* row = S + (size_t)blockIdx.x * max_seq;
+    float* row = S + blockIdx.y * sc_ld + (size_t)blockIdx.x * max_seq;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     // zero the positions past the row that the chains read
     for (int i = tid; i < 8 * LDT; i += SMX_NT) (&tr[0][0])[i] = 0.0f;
@@ -627,16 +640,24 @@ DEV float pvd_chunk(float (*Vt)[64 / G][PVD_LD], float (*Pt)[G][PVD_LD], int h, 
 // Waits until at most N vector-memory operations of this wave are in flight.
 #define PVD_VMCNT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
 
-template <int HD, int G, bool Q8>
+// MS: one token of each of gridDim.z sessions (no warm-up workgroups).
+template <int HD, int G, bool Q8, bool MS>
 __global__ __launch_bounds__(192) void k_attn_pvd(const float* __restrict__ P, const float* __restrict__ vc,
                                                   const int32_t* __restrict__ pos0p, int n_kv, int max_seq,
-                                                  float* __restrict__ out, DpufKvQ8 c8, DpufWarm warm) {
+                                                  float* __restrict__ out, DpufKvQ8 c8, DpufWarm warm, MsTab ms) {
+    static_assert(!MS || !Q8, "sessions: the fp32 cache");
     using S = PvdShape<G, Q8>;
     constexpr int DW = S::DW;
     static_assert(G == 2 || G == 4, "every 16-lane row of the chain wave holds one head");
     __shared__ __align__(16) float Vt[3][DW][PVD_LD];
     __shared__ __align__(16) float Pt[3][G][PVD_LD];
-    const int L = *pos0p + 1, nck = (L + PVD_CK - 1) / PVD_CK, nfull = L / PVD_CK;
+    const int z = MS ? blockIdx.z : 0;
+    const int L = pos0p[z] + 1, nck = (L + PVD_CK - 1) / PVD_CK, nfull = L / PVD_CK;
+    if (MS) {
+        P += (size_t)z * ms.sc_ld;
+        vc = ms.vcs[z] + ms.lo;
+        out += (size_t)z * ms.q_ld;
+    }
     if ((int)blockIdx.y >= HD / DW) {
         // warm-up workgroups (after the chain workgroups in dispatch order)
         const int wi = ((int)blockIdx.y - HD / DW) * n_kv + (int)blockIdx.x;
@@ -744,7 +765,7 @@ __global__ __launch_bounds__(192) void k_attn_pvd(const float* __restrict__ P, c
 // workgroup per remaining CU (a multiple of 8) warms the V rows (base, rb
 // bytes per row) into the L2 that reads them.
 static void smx_launch(void* s, int seg, float* scores, const int32_t* pos0p, int max_seq, int n_q, int n_kv, int G,
-                       const void* vbase, int rb) {
+                       const void* vbase, int rb, int n_ses = 1, size_t sc_ld = 0) {
     SmxWarm W{nullptr, rb, n_kv, n_q};
     int nwarm = 0;
     if (PVD_SMX_WARM && (G == 2 || G == 4) && n_kv % 8 == 0 && vbase) {
@@ -752,9 +773,9 @@ static void smx_launch(void* s, int seg, float* scores, const int32_t* pos0p, in
         if (nwarm > 0) W.base = (const uint8_t*)vbase;
         else nwarm = 0;
     }
-    const dim3 g(n_q + nwarm);
+    const dim3 g(n_q + nwarm, n_ses);
 #define SMX_CASE(SG) \
-    if (seg == SG) hipLaunchKernelGGL(k_attn_smx<SG>, g, dim3(SMX_NT), 0, ST(s), scores, pos0p, max_seq, W);
+    if (seg == SG) hipLaunchKernelGGL(k_attn_smx<SG>, g, dim3(SMX_NT), 0, ST(s), scores, pos0p, max_seq, W, sc_ld);
     SMX_CASE(16) SMX_CASE(32) SMX_CASE(48) SMX_CASE(64) SMX_CASE(80) SMX_CASE(96) SMX_CASE(128)
 #undef SMX_CASE
 }
@@ -780,11 +801,11 @@ static void pv_wide_launch(void* s, int G, int gm, const float* scores, const fl
             rows = (n_cu / n_kv > ns ? n_cu / n_kv : ns) - ns;
         }
         if (G == 4)
-            hipLaunchKernelGGL((k_attn_pvd<HD, 4, Q8>), dim3(n_kv, ns + rows), dim3(192), 0, ST(s), scores, vc, pos0p,
-                               n_kv, max_seq, out, c8, warm);
+            hipLaunchKernelGGL((k_attn_pvd<HD, 4, Q8, false>), dim3(n_kv, ns + rows), dim3(192), 0, ST(s), scores, vc, pos0p,
+                               n_kv, max_seq, out, c8, warm, MsTab{});
         else
-            hipLaunchKernelGGL((k_attn_pvd<HD, 2, Q8>), dim3(n_kv, ns + rows), dim3(192), 0, ST(s), scores, vc, pos0p,
-                               n_kv, max_seq, out, c8, warm);
+            hipLaunchKernelGGL((k_attn_pvd<HD, 2, Q8, false>), dim3(n_kv, ns + rows), dim3(192), 0, ST(s), scores, vc, pos0p,
+                               n_kv, max_seq, out, c8, warm, MsTab{});
     }
     else if (gm == 2)
         hipLaunchKernelGGL((k_attn_pvw<HD, 2, Q8>), dim3(n_kv, HD / 4), dim3(192), 0, ST(s), scores, vc, pos0p, n_q,
@@ -820,11 +841,11 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
         const dim3 g1s(n_kv, (lmax + AS_KC - 1) / AS_KC);                                                         \
         const size_t l1s = (size_t)(AS_KC * (HDV + 8) + GMV * HDV) * 4;                                           \
         if (rope)                                                                                                 \
-            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, true>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q, n_kv, \
-                               max_seq, scale, scores, *rope);                                                    \
+            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, true, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q, n_kv, \
+                               max_seq, scale, scores, *rope, MsTab{});                                                    \
         else                                                                                                      \
-            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q,      \
-                               n_kv, max_seq, scale, scores, ScRope{});                                           \
+            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, false, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q,      \
+                               n_kv, max_seq, scale, scores, ScRope{}, MsTab{});                                           \
     }
 #define WIDE_LAUNCH(HDV)                                                                                          \
     if (gm == 2) SC1_LAUNCH(HDV, 2) else if (gm == 4) SC1_LAUNCH(HDV, 4) else SC1_LAUNCH(HDV, 8)                  \
@@ -845,6 +866,51 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
         }
     }
     return -1;
+}
+
+// One token of each of n sessions over an fp32 cache, each against its own
+// slot's cache (tables kcs / vcs, positions pos), in the three launches of the
+// longest session alone: QK-norm, RoPE, KV store and scores; softmax; P.V.
+// One by one, five sessions of 200 to 2 600 keys took 15 launches and 85 us per
+// layer at the 8B width; together 33.  Every session takes the kernels it would take
+// alone, so its results are the same bits.  Groups of 2 and 4; -1 with nothing
+// launched otherwise.
+int32_t attn_wide_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v, const float* qn,
+                           const float* kn, float eps, const float* cos_tab, const float* sin_tab, float* const* kcs,
+                           float* const* vcs, size_t lo, float* out, float* scores, const int32_t* pos, int32_t n_q,
+                           int32_t n_kv, int32_t hd, int32_t max_seq, float scale) {
+    if (n_kv <= 0 || n_q % n_kv || (hd != 64 && hd != 128 && hd != 256)) return -1;
+    const int G = n_q / n_kv;
+    if (G != 2 && G != 4) return -1;
+    if (lmax > max_seq) lmax = max_seq;
+    const int segs[7] = {16, 32, 48, 64, 80, 96, 128};
+    int seg = 0;
+    for (int i = 0; i < 7 && !seg; i++)
+        if (64 * segs[i] >= lmax) seg = segs[i];
+    if (!seg) return -1;
+    const ScRope r = {k, v, qn, kn, eps, cos_tab, sin_tab, NULL, NULL};
+    const MsTab ms = {kcs, vcs, lo, n_q * hd, n_kv * hd, (size_t)n_q * max_seq};
+    const dim3 g1(n_kv, (lmax + AS_KC - 1) / AS_KC, n);
+#define MS_LAUNCH(HDV, GV)                                                                                         \
+    {                                                                                                              \
+        const size_t l1 = (size_t)(AS_KC * (HDV + 8) + GV * HDV) * 4;                                              \
+        hipLaunchKernelGGL((k_attn_sc1<HDV, GV, true, true>), g1, dim3(256), l1, ST(s), q, NULL, pos, n_q, n_kv,   \
+                           max_seq, scale, scores, r, ms);                                                         \
+        smx_launch(s, seg, scores, pos, max_seq, n_q, n_kv, G, nullptr, 0, n, ms.sc_ld);                           \
+        hipLaunchKernelGGL((k_attn_pvd<HDV, GV, false, true>), dim3(n_kv, HDV * GV / 64, n), dim3(192), 0, ST(s),  \
+                           scores, NULL, pos, n_kv, max_seq, out, DpufKvQ8{}, DpufWarm{}, ms);                     \
+    }
+    if (hd == 64) {
+        if (G == 2) MS_LAUNCH(64, 2) else MS_LAUNCH(64, 4)
+    } else if (hd == 128) {
+        if (G == 2) MS_LAUNCH(128, 2) else MS_LAUNCH(128, 4)
+    } else {
+        if (G == 2) MS_LAUNCH(256, 2) else MS_LAUNCH(256, 4)
+    }
+#undef MS_LAUNCH
+    LAUNCHED("k_attn sessions");
+    for (int i = 0; i < n; i++) attn_path_note(1);
+    return 0;
 }
 
 int32_t attn_wide_q8(void* s, int32_t lmax, const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd,

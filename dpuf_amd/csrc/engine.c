@@ -886,24 +886,38 @@ static DpufWarm attn_warm_fed_o(Engine* e, const LayerJobs* lj, const LayerJobs*
 }
 
 /* Attention of a multi-session step at layer l (ms_n = M tokens, one per
- * session): the first ms_short tokens (fp32 cache, short context) in one
- * fused decode launch over their sessions' caches; every other token alone,
- * at its own position against its own slot's cache, through the one-token
- * kernels a single-session step of that length takes (dpuf_engine.c:1404-1600
- * serves each slot's sequence the same way); then, when any token took the
- * latter, the O-input prep of all M rows (the fused kernel's rows prep to the
- * same values). */
+ * session): when every context is short (the first ms_short = M tokens, fp32
+ * cache), one fused decode launch over the sessions' caches.  When some are
+ * longer (fp32 cache, groups of 2 or 4), all of them together through the
+ * one-token kernels of long contexts with a session axis: the short ones end
+ * long before the longest, while the fused launch for them was 16 us more per
+ * layer.  Otherwise the short ones fused and every other token alone, at its
+ * own position against its own slot's cache, through the one-token kernels a
+ * single-session step of that length takes (dpuf_engine.c:1404-1600 serves
+ * each slot's sequence the same way).  Unless all went fused, the O-input prep
+ * of all M rows follows (the fused kernel's rows prep to the same values). */
 static void enqueue_ms_attention(Engine* e, int32_t l, int32_t M, float eps, float scale, const uint8_t* o_sign) {
     void* s = e->stream;
     const DpufWarm no_warm = {0};
     const size_t lo = (size_t)l * e->nkv * e->max_seq * e->hd;
     const int32_t ns = e->ms_short;
     const float *qn = e->d_norm[4 * l + 1], *kn = e->d_norm[4 * l + 2];
-    if (ns > 0)
+    int32_t done = 0;
+    if (!is_q8(e) && ns < M && M > 1) {
+        int32_t lmax = 0;
+        for (int32_t m = 0; m < M; m++) lmax = e->ms_pos[m] + 1 > lmax ? e->ms_pos[m] + 1 : lmax;
+        if (dpuf_hip_attn_sessions(s, M, lmax, e->q, e->k, e->v, qn, kn, eps, e->d_cos, e->d_sin, e->d_ms_kc,
+                                   e->d_ms_vc, lo, e->ao, e->scores, e->d_ms_pos, e->nq, e->nkv, e->hd, e->max_seq,
+                                   scale) == 0)
+            done = M;
+    }
+    if (!done && ns > 0) {
         dpuf_hip_attn_dec(s, ns, e->q, e->k, e->v, qn, kn, eps, e->d_cos, e->d_sin, NULL, NULL, e->d_ms_pos, e->nq,
                           e->nkv, e->hd, e->max_seq, scale, e->ao, o_sign, e->prep[0], e->d_ms_kc, e->d_ms_vc, lo,
                           no_warm);
-    for (int32_t m = ns; m < M; m++) {
+        done = ns;
+    }
+    for (int32_t m = done; m < M; m++) {
         float* q = e->q + (size_t)m * e->qd;
         float* k = e->k + (size_t)m * e->kvd;
         float* v = e->v + (size_t)m * e->kvd;

@@ -252,6 +252,14 @@ int32_t dpuf_hip_attn_dec(void* s, int32_t M, const float* q, const float* k, co
                           float* vc, const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq,
                           float scale, float* ao, const uint8_t* o_sign, DpufPrep op, float* const* kcs,
                           float* const* vcs, size_t l_off, DpufWarm warm);
+/* One token of each of n sessions (lmax: the longest session's keys), fp32 caches kcs[m] + l_off / vcs[m] + l_off,
+ * rows m of q, k, v and out: QK-norm, RoPE, KV store and attention.  -1 with
+ * nothing launched when the shape has no such kernels. */
+int32_t dpuf_hip_attn_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v,
+                               const float* qn, const float* kn, float eps, const float* cos_tab, const float* sin_tab,
+                               float* const* kcs, float* const* vcs, size_t l_off, float* out, float* scores,
+                               const int32_t* pos, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq,
+                               float scale);
 /* Attention launches enqueued per path (dpuf_amd_attn_path_count); -1 for
  * another `which`. */
 #define DPUF_HIP_ATTN_PATHS 6
