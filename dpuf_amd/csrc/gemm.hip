@@ -41,9 +41,14 @@
 //     element: |16 (D - sum8)| < 2^20 stays inside that binade, so the result
 //     read as a float is 1 / (2 pi) + n 2^-26 exactly and one exact
 //     subtraction gives n 2^-26 at full rate (v_cvt_f32_i32 issues at half);
+//   * mode 12's products ws * xs come from 4 x 4 outer-product MFMAs (one for
+//     256 outputs in place of 4 v_mul_f32; gm_outer4), issued with the dots
+//     before any result is read: the chains are left with one subtraction and
+//     one FMA per output.  (With the products on the vector unit down M = 29
+//     32 us, 27 so, M = 512 119 and 108.  Left to the compiler's order, which
+//     waits for each product in turn, they gained nothing.)
 //   * weight scales are widened to float once per workgroup when they are
-//     staged, so the product with xs is a v_mul_f32 (v_fma_mix_f32 issues at
-//     half rate).
+//     staged (v_fma_mix_f32 issues at half rate).
 // acc carries the factor 2^-22 (modes 13 / 14, whose u needs no offset:
 // 2^-26), removed at the end: powers of two commute with every rounding here
 // as long as no partial sum is below 2^-104 in magnitude.
@@ -60,9 +65,9 @@
 // e; D lane l = column l % 32, rows 8 (v / 4) + 4 (l / 32) + v % 4.
 //
 // us per launch at the 8B widths, before (one 16-row x 64-token fp16 tile per
-// wave for every M) -> now: down M = 29 85 -> 32, M = 90 93 -> 43, M = 512 144
-// -> 119; O 30 -> 13, 31 -> 17, 47.5 -> 38; mode 14 down M = 90 135 -> 51, M =
-// 512 223 -> 146; gate + up with the SwiGLU M = 29 46 -> 32, M = 512 204 -> 178.
+// wave for every M) -> now: down M = 29 85 -> 27, M = 90 93 -> 37, M = 512 144
+// -> 108; O 30 -> 11, 31 -> 15, 47.5 -> 39; mode 14 down M = 90 135 -> 48, M =
+// 512 223 -> 145; gate + up M = 512 225 -> 181.
 // ---------------------------------------------------------------------------
 
 #define GM_SWI_ROWS 16384  // gate + up rows from which the fused SwiGLU launch pays
@@ -127,6 +132,14 @@ DEV gm_h8 gm_unpack_a_asym(uint32_t w, uint32_t h) {
 
 
 // ---------------------------------------------------------------------------
+// Sixteen 4 x 4 outer products a b^T in one fp32 MFMA, each product rounded
+// once (the FMA's addend is +0: a product of zero may lose its sign, which
+// cannot reach an accumulator that is never -0): lane l = (block l / 4, column
+// l % 4) gives a for row l % 4 and b for its column, and gets the block's 4 rows.
+DEV gm_f4 gm_outer4(float a, float b) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+}
+
 // k_gemm_mfma: NW waves of 16 rows each, TT 16-token tiles per workgroup, for
 // launches with few tiles: a wave of one tile (TT = 1) leaves the most waves,
 // and a tile's serial chain over K is then all of the launch's length.
@@ -308,7 +321,7 @@ k_gemm_mfma(GmArgs A) {
     // LDS operands of G blocks, read one set ahead of their MFMAs; the token
     // scales (and xm_s) of a quad are read with its first set
     long bf[2][G][TT];
-    float wsr[2][G][4];
+    float wsr[2][G][ASYM ? 4 : 1];
     gm_i4 c0 = {(int)BASE, (int)BASE, (int)BASE, (int)BASE};
     asm("" : "+v"(c0));  // loop-invariant registers
     float xs[2][TT][4];
@@ -316,9 +329,13 @@ k_gemm_mfma(GmArgs A) {
     auto lds_set = [&](int buf, int b, int slot, int xslot) {
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const gm_f4 y = *(const gm_f4*)&bw[buf][b + g][16 * w + 4 * kc];
+            if (ASYM) {
+                const gm_f4 y = *(const gm_f4*)&bw[buf][b + g][16 * w + 4 * kc];
 #pragma unroll
-            for (int v = 0; v < 4; v++) wsr[slot][g][v] = y[v];
+                for (int v = 0; v < 4; v++) wsr[slot][g][ASYM ? v : 0] = y[v];
+            } else {
+                wsr[slot][g][0] = bw[buf][b + g][16 * w + 4 * kc + (l & 3)];
+            }
 #pragma unroll
             for (int t = 0; t < TT; t++) bf[slot][g][t] = *(const long*)&bq[buf][b + g][32 * (16 * t + i16) + 8 * kc];
         }
@@ -353,17 +370,10 @@ k_gemm_mfma(GmArgs A) {
             th[3] = th[2] >> 4;
             skp_transpose(th[0], th[1], th[2], th[3]);
         }
+        // the quad's weight operands
+        long wa[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int slot = G == 4 ? x : (j / G) & 1, g = j % G;
-            if (g == 0) {
-                // the set after this one
-                if (j + G < 4)
-                    lds_set(buf, b + j + G, slot ^ 1, x);
-                else if (more)
-                    lds_set(buf, b + 4, slot ^ 1, x ^ 1);
-            }
-            if (j >= nb) break;  // uniform
             uint32_t lo, hi;
             if (!ASYM) {
                 // 16 (u - 8) as int8: the nibble with its top bit flipped, in
@@ -378,41 +388,64 @@ k_gemm_mfma(GmArgs A) {
                     hi |= (th[j] << 2) & 0x30303030u;
                 }
             }
-            const long a = (long)(((uint64_t)hi << 32) | lo);
-            const float(&ws)[4] = wsr[slot][g];
+            wa[j] = (long)(((uint64_t)hi << 32) | lo);
+        }
+        // G blocks at a time: their dots (and mode 12's products) are all
+        // issued before the first is read, so their latencies overlap
 #pragma unroll
-            for (int t = 0; t < TT; t++) {
-                const gm_i4 di = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bf[slot][g][t], c0, 0, 0, 0);
-                const float sx = xs[x][t][j];
-                float d[4];
+        for (int j0 = 0; j0 < 4; j0 += G) {
+            const int slot = G == 4 ? x : (j0 / G) & 1;
+            // the set after this one
+            if (j0 + G < 4)
+                lds_set(buf, b + j0 + G, slot ^ 1, x);
+            else if (more)
+                lds_set(buf, b + 4, slot ^ 1, x ^ 1);
+            if (j0 >= nb) break;  // uniform
+            gm_i4 di[G][TT];
+            gm_f4 pr[G][TT];
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int di_v = di[v];
-                    d[v] = __builtin_bit_cast(float, di_v) - __builtin_bit_cast(float, BASE);
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int t = 0; t < TT; t++) {
+                    di[g][t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wa[j0 + g], bf[slot][g][t], c0, 0, 0, 0);
+                    // rows 4 kc + 0 .. 3, the lane's token
+                    if (!ASYM) pr[g][t] = gm_outer4(wsr[slot][g][0], xs[x][t][j0 + g]);
                 }
-                if (!ASYM) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const int j = j0 + g;
+                if (j >= nb) break;  // uniform
+#pragma unroll
+                for (int t = 0; t < TT; t++) {
+                    const float sx = xs[x][t][j];
+                    float d[4];
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
-                        const float p = ws[v] * sx;
-                        acc[t][v] = fmaf(d[v], p, acc[t][v]);
+                        const int di_v = di[g][t][v];
+                        d[v] = __builtin_bit_cast(float, di_v) - __builtin_bit_cast(float, BASE);
                     }
-                } else if ((j & 1) == 0) {
+                    if (!ASYM) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++) dk[t][v] = d[v];
-                } else {
-                    const float sx0 = xs[x][t][j - 1], sm_ = xm[x][t][j >> 1];
+                        for (int v = 0; v < 4; v++) acc[t][v] = fmaf(d[v], pr[g][t][v], acc[t][v]);
+                    } else if ((j & 1) == 0) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const float p1 = d[v] * sx;
-                        const float fd = fmaf(dk[t][v], sx0, p1);
-                        acc[t][v] = fmaf(fd, dsk[v], acc[t][v]);
-                        acc[t][v] = fmaf(ws[v], sm_, acc[t][v]);
+                        for (int v = 0; v < 4; v++) dk[t][v] = d[v];
+                    } else {
+                        const float sx0 = xs[x][t][j - 1], sm_ = xm[x][t][j >> 1];
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const float p1 = d[v] * sx;
+                            const float fd = fmaf(dk[t][v], sx0, p1);
+                            acc[t][v] = fmaf(fd, dsk[v], acc[t][v]);
+                            acc[t][v] = fmaf(wsr[slot][g][ASYM ? v : 0], sm_, acc[t][v]);
+                        }
                     }
                 }
-            }
-            if (ASYM && (j & 1) == 0) {
+                if (ASYM && (j & 1) == 0) {
 #pragma unroll
-                for (int v = 0; v < 4; v++) dsk[v] = ws[v];
+                    for (int v = 0; v < 4; v++) dsk[v] = wsr[slot][g][ASYM ? v : 0];
+                }
             }
         }
     };
@@ -656,8 +689,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
         } else {
 #pragma unroll
             for (int k = 0; k < SPT; k++) {
-                const int i = tid + 256 * k;
-                xl[buf][i % SB][i / SB] = ss[k];
+                const int i = tid + 256 * k, t = i / SB;
+                xl[buf][i % SB][(t & 32) + ((t >> 2) & 1) * 16 + (t & 3) * 4 + ((t >> 3) & 3)] = ss[k];
             }
         }
         if (tid < WS) {
@@ -679,15 +712,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
 
     // LDS operands of one block
     gm_i4 af[2];
-    float xs[2][16];
+    float xs[2][ASYM ? 16 : 4];
     float ws[2][RF];
     auto lds_blk = [&](int buf, int b, int slot) {
         af[slot] = *(const gm_i4*)&aq[buf][b][32 * (32 * wt + r32) + 16 * h];
+        if (ASYM) {
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const gm_f4 x = *(const gm_f4*)&xl[buf][b][32 * wt + 8 * g + 4 * h];
+            for (int g = 0; g < 4; g++) {
+                const gm_f4 x = *(const gm_f4*)&xl[buf][b][32 * wt + 8 * g + 4 * h];
 #pragma unroll
-            for (int v = 0; v < 4; v++) xs[slot][4 * g + v] = x[v];
+                for (int v = 0; v < 4; v++) xs[slot][ASYM ? 4 * g + v : 0] = x[v];
+            }
+        } else {
+            // tokens 8 g + 4 h + l % 4, g = 0 .. 3
+            const gm_f4 x = *(const gm_f4*)&xl[buf][b][32 * wt + 16 * h + 4 * (l & 3)];
+#pragma unroll
+            for (int g = 0; g < 4; g++) xs[slot][g] = x[g];
         }
 #pragma unroll
         for (int f = 0; f < RF; f++) ws[slot][f] = wl[buf][b][(SWI ? 64 * f + 32 * wr : 32 * (RF * wr + f)) + r32];
@@ -745,6 +785,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
             for (int f = 0; f < RF; f++) {
                 d[f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[b], wa[b][f], c0, 0, 0, 0);
             }
+            // products xs ws of tokens 8 g + 4 h + 0 .. 3 and the lane's row, all
+            // issued before the first dot is read: their latencies overlap
+            gm_f4 pr[RF][4];
+            if (!ASYM) {
+#pragma unroll
+                for (int f = 0; f < RF; f++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) pr[f][g] = gm_outer4(xs[b][g], ws[b][f]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int f = 0; f < RF; f++) {
                 if (!ASYM) {
@@ -752,15 +802,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
                     for (int v = 0; v < 16; v++) {
                         const int di = d[f][v];
                         const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
-                        const float pr = xs[b][v] * ws[b][f];
-                        acc[f][v] = fmaf(x, pr, acc[f][v]);
+                        acc[f][v] = fmaf(x, pr[f][v >> 2][v & 3], acc[f][v]);
                     }
                 } else if (b == 0) {
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
                         const int di = d[f][v];
                         dk[f][v] = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
-                        xk[v] = xs[0][v];
+                        xk[v] = xs[0][ASYM ? v : 0];
                     }
                     dd[f] = ws[0][f];
                 } else {
@@ -768,7 +817,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
                     for (int v = 0; v < 16; v++) {
                         const int di = d[f][v];
                         const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
-                        const float p1 = x * xs[1][v];
+                        const float p1 = x * xs[1][ASYM ? v : 0];
                         const float fd = fmaf(dk[f][v], xk[v], p1);
                         acc[f][v] = fmaf(fd, dd[f], acc[f][v]);
                     }
@@ -1598,7 +1647,7 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
         }
         // The tile by the number of 16 x 16 tiles per SIMD (each a serial
         // chain over K).  Measured, us (16 x 16 | 16 x 32 | 32 x 32 | 64 x 32
-        // per wave), mode 12: 4 096 rows, K = 12 288: 2 per SIMD 43 | 61 | 88 |
+        // per wave; before the outer-product MFMAs), mode 12: 4 096 rows, K = 12 288: 2 per SIMD 43 | 61 | 88 |
         // 126; 4 per SIMD 86 | 81 | 90 | 126; 8 per SIMD 179 | 160 | 119 | 136.
         // 6 144 rows, K = 4 096: 3 per SIMD 26 | 29 | 32 | 46; 6 per SIMD 46 |
         // 39 | 37 | 47.  24 576 rows: 12 per SIMD 86 | 72 | 52 | 62; 48 per SIMD
