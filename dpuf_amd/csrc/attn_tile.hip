@@ -335,8 +335,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 //     memory: lane (c, g) reads dims 32 w + 2 c, + 1 of key 4 i + g, 128
 //     contiguous bytes per key, 8 steps ahead of their MFMAs.
 // RES: every chunk keeps its LDS slot and pass B reads pass A's e; otherwise
-// (rows too long for that) pass B loads the scores and forms e again, in two
-// rotating slots.  A slot is [row][key % 4][key / 4 (+ 4 padding)], so four
+// (rows too long for that) pass A stores e over the scores and pass B loads it
+// (each thread its own elements), in two rotating slots.  A slot is [row][key % 4][key / 4 (+ 4 padding)], so four
 // steps' A operands are one 16-byte read.  Keys from Lmin & ~3 on (at most
 // qt + 2) are reached by some rows only and take one predicated FMA per
 // output on the vector unit, so a masked key never multiplies V.
@@ -360,7 +360,7 @@ struct PvmGeo {
 
 template <int HD, bool Q8, bool RES>
 __global__ __launch_bounds__(2 * HD) void k_attn_pvm(
-    const float* __restrict__ S, const float* __restrict__ smax, const float* __restrict__ vc, DpufKvQ8 c8,
+    float* S, const float* __restrict__ smax, const float* __restrict__ vc, DpufKvQ8 c8,
     const int32_t* __restrict__ pos0p, int M, int n_q, int n_kv, int max_seq, int qt, int tpw,
     float* __restrict__ out, const uint8_t* __restrict__ o_sign, DpufPrep op) {
     using P = PvmGeo<HD>;
@@ -399,14 +399,33 @@ __global__ __launch_bounds__(2 * HD) void k_attn_pvm(
         for (int o = NI / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     }
     float* const eo = sm + tr * RS + ti;
-    auto e_store = [&](int ch, int sl, gm_f4 x) {
-        const int t = ch * KC + 4 * ti;
+    auto l_store = [&](int sl, gm_f4 v) {
         float* e = eo + sl * P::SLOT;
 #pragma unroll
+        for (int k = 0; k < 4; k++) e[k * GS] = v[k];
+    };
+    auto e_store = [&](int ch, int sl, gm_f4 x) {
+        const int t = ch * KC + 4 * ti;
+        gm_f4 v;
+#pragma unroll
         for (int k = 0; k < 4; k++) {
-            float v = exp_poly(x[k] - mx);
-            if (t + k >= n8t) v = t + k < Lt ? expf_libc(x[k] - mx) : 0.0f;
-            e[k * GS] = v;
+            v[k] = exp_poly(x[k] - mx);
+            if (t + k >= n8t) v[k] = t + k < Lt ? expf_libc(x[k] - mx) : 0.0f;
+        }
+        l_store(sl, v);
+        if (!RES && Lt > 0) {
+            // the thread's own scores again, for its pass B
+            if (t + 3 < max_seq) {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(gm_u4, v), rS, so + (uint32_t)(ch * KC * 4), 0, 0);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float vk = v[k];
+                    if (t + k < max_seq)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, vk), rS,
+                                                              so + (uint32_t)(ch * KC * 4) + 4 * k, 0, 0);
+                }
+            }
         }
     };
 
@@ -508,7 +527,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_pvm(
         if (!RES) {
             const gm_f4 x = xn;
             xn = s_load(ch + 1);
-            e_store(ch, sl, x);
+            l_store(sl, x);  // past a row's kv_len: never used
             __syncthreads();
         }
         const float* ps = pa + sl * P::SLOT;
