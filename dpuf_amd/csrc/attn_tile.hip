@@ -342,12 +342,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // output on the vector unit, so a masked key never multiplies V.
 // Bound: fp32 matrix rate, then exp on the vector unit.  Measured at the 8B
 // geometry against the vector kernels (softmax + P.V with the chains as FMAs
-// from LDS): 256 tokens at 4 096 keys 1 433 -> 163 us (streamed), 512 tokens
+// from LDS): 256 tokens at 4 096 keys 1 433 -> 143 us (streamed), 512 tokens
 // from an empty cache 48.0 -> 31.0 (resident), 29 tokens at 439 keys 40.3 ->
-// 18.5, int8 cache with 90 tokens at 790 keys 86.9 + 5.0 (its O prep) -> 29.6.
+// 17.2, int8 cache with 90 tokens at 790 keys 86.9 + 5.0 (its O prep) -> 27.7.
 // Resident rows up to 76 KB of LDS: two workgroups per CU; past that one
 // workgroup per CU would leave the matrix cores to four waves, and streaming
-// costs one more exp per score (about a fifth of the MFMA time).
+// costs each score a store and a load.
 // ---------------------------------------------------------------------------
 template <int HD>
 struct PvmGeo {
@@ -477,15 +477,31 @@ __global__ __launch_bounds__(2 * HD) void k_attn_pvm(
         uint16_t b[Q8 ? VS : 1];
         float s[Q8 ? VS : 1];
     };
+    // Buffer loads with the step in the scalar offset: no vector instruction
+    // per load (they add to the MFMAs' time).  A step past the cache's last
+    // whole one (never used) repeats that; the scalar offset is outside the
+    // descriptor's range check, which covers the lane offsets of caches of
+    // fewer than four rows.
+    constexpr int VB1 = Q8 ? 1 : 4;  // bytes per element
+    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
+        Q8 ? (void*)(c8.vq + (size_t)kvh * max_seq * HD) : (void*)(vc + (size_t)kvh * max_seq * HD), 0,
+        max_seq * HD * VB1, ATL_RSRC3);
+    const __amdgpu_buffer_rsrc_t rVs = __builtin_amdgcn_make_buffer_rsrc(
+        Q8 ? (void*)(c8.vs + (size_t)kvh * max_seq * NB) : (void*)S, 0, max_seq * NB * 4, ATL_RSRC3);
+    const uint32_t vo = (uint32_t)(g * HD + d0) * VB1, vso = (uint32_t)(g * NB + w) * 4u;
+    const int slast = max(max_seq / 4 - 1, 0);
     auto v_load = [&](int step, VB& B) {
 #pragma unroll
         for (int i = 0; i < VS; i++) {
-            const int t = min(4 * (step + i) + g, max_seq - 1);
+            const int st = min(step + i, slast);
             if (Q8) {
-                B.b[i] = *(const uint16_t*)(Vq + (size_t)t * HD);
-                B.s[i] = Vsc[(size_t)t * NB];
+                B.b[i] = __builtin_amdgcn_raw_buffer_load_b16(rV, vo, st * 4 * HD, 0);
+                const uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(rVs, vso, st * 16 * NB, 0);
+                B.s[i] = __builtin_bit_cast(float, x);
             } else {
-                B.v[i] = *(const float2*)(Vh + (size_t)t * HD);
+                const gm_u2 x = __builtin_bit_cast(gm_u2, __builtin_amdgcn_raw_buffer_load_b64(rV, vo, st * 16 * HD, 0));
+                const uint32_t x0 = x[0], x1 = x[1];
+                B.v[i] = make_float2(__builtin_bit_cast(float, x0), __builtin_bit_cast(float, x1));
             }
         }
     };
