@@ -81,7 +81,7 @@ DEV void score_max_slot(float mx, int L, float* slot, int g) {
 // fp32 MFMAs and vector instructions do not overlap).
 // Every wave writes the maximum of its keys per row to smax[row][slot].
 // Measured, 32 heads of 128 over 8 KV heads, against the vector kernel
-// k_attn_sc it replaces here: 256 tokens at 4 096 keys 168 -> 112 us (53 us
+// k_attn_sc it replaces here: 256 tokens at 4 096 keys 168 -> 102 us (53 us
 // at the matrix rate), 512 tokens from an empty cache 30.6 -> 26.0, 29 tokens
 // at 439 keys 7.8 -> 5.7.
 // ---------------------------------------------------------------------------
@@ -634,10 +634,12 @@ static void launch(void* s, int M, int lmax, const float* q, const float* kc, co
     constexpr int XT = HD == 256 || Q8 ? 1 : 2;
     const int G = n_q / n_kv, qs = 16 * XT / G, qp = 16 / G;
     // key tiles per wave: as many as keep about two waves per SIMD, at most
-    // 8 (128 keys), and enough for ATL_SLOTS slots to cover the keys
+    // 32 (512 keys: a wave's start, its q rows and first K tile, is paid once;
+    // 256 tokens at 4 096 keys 111 us with at most 8, 102 so), and enough for
+    // ATL_SLOTS slots to cover the keys
     const int kt = (lmax + 15) / 16, rt = (M + qs - 1) / qs;
     long long tpw = (long long)kt * rt * n_kv / (8 * dpuf_hip_cu_count());
-    tpw = tpw < 1 ? 1 : tpw > 8 ? 8 : tpw;
+    tpw = tpw < 1 ? 1 : tpw > 32 ? 32 : tpw;
     if (tpw * ATL_SLOTS < kt) tpw = (kt + ATL_SLOTS - 1) / ATL_SLOTS;
     const dim3 g1(n_kv, rt, (unsigned)((kt + 4 * tpw - 1) / (4 * tpw)));
     if (Q8)
