@@ -39,11 +39,12 @@
 // distinct banks.
 
 
-// MS: one token of each of gridDim.z sessions (ROPE only).
+typedef __attribute__((address_space(1))) float* glb_f;
+
+// MS: one token of each of gridDim.z sessions (ROPE only; k_attn_sc1_ms).
 template <int HD, int GM, bool ROPE, bool MS>
-__global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, const float* __restrict__ kc,
-                                                  const int32_t* __restrict__ pos0p, int n_q, int n_kv, int max_seq,
-                                                  float scale, float* __restrict__ S, ScRope ra, MsTab ms) {
+DEV void sc1_body(const float* __restrict__ q, const float* __restrict__ kc, const int32_t* __restrict__ pos0p, int n_q,
+                  int n_kv, int max_seq, float scale, float* __restrict__ S, const ScRope& ra, const MsTab& ms) {
     static_assert(!MS || ROPE, "sessions take the RoPE in the launch");
     constexpr int LD = HD + 8, E = HD / 64;
     extern __shared__ __align__(16) float sm[];
@@ -54,13 +55,14 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
     const int z = MS ? blockIdx.z : 0;
     const int pos = pos0p[z], L = pos + 1;
     if (t0 >= L) return;  // every key of the chunk is past the row
+    const float* rk = ROPE ? ra.k + (MS ? (size_t)z * ms.kv_ld : 0) : nullptr;
+    const float* rv = ROPE ? ra.v + (MS ? (size_t)z * ms.kv_ld : 0) : nullptr;
+    // global pointers: a table's would make these flat accesses
+    const glb_f rkc = (glb_f)(MS ? ms.kcs[z] + ms.lo : ra.kc);
+    const glb_f rvc = (glb_f)(MS ? ms.vcs[z] + ms.lo : ra.vc);
+    const glb_f kg = MS ? rkc : (glb_f)kc;
     if (MS) {
         q += (size_t)z * ms.q_ld;
-        ra.k += (size_t)z * ms.kv_ld;
-        ra.v += (size_t)z * ms.kv_ld;
-        ra.kc = ms.kcs[z] + ms.lo;
-        ra.vc = ms.vcs[z] + ms.lo;
-        kc = ra.kc;
         S += (size_t)z * ms.sc_ld;
     }
     // ROPE units of wave tid / 64: q rows u < GM, then (if this chunk holds
@@ -72,12 +74,13 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
     float vv[E];
     {
         constexpr int NK = AS_KC * (HD / 4) / 256, NQ = (GM * (HD / 4) + 255) / 256;
-        float4 kx[NK], qx[NQ];
+        gm_f4 kx[NK];
+        float4 qx[NQ];
 #pragma unroll
         for (int k = 0; k < NK; k++) {
             const int e = tid + 256 * k, kr = e / (HD / 4), c = e % (HD / 4);
             const int t = t0 + kr < max_seq ? t0 + kr : max_seq - 1;
-            kx[k] = *(const float4*)(kc + ((size_t)kvh * max_seq + t) * HD + 4 * c);
+            kx[k] = *(const __attribute__((address_space(1))) gm_f4*)(kg + ((size_t)kvh * max_seq + t) * HD + 4 * c);
         }
         if (ROPE) {
 #pragma unroll
@@ -87,9 +90,9 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
                     const int hr = u < G ? u : G - 1;  // rows past the group repeat the last head (never written)
                     qk_head_load<HD>(q + ((size_t)kvh * G + hr) * HD, ra.qn, ra.cos_tab, ra.sin_tab, pos, lane, hu[k]);
                 } else if (u < nu) {
-                    qk_head_load<HD>(ra.k + (size_t)kvh * HD, ra.kn, ra.cos_tab, ra.sin_tab, pos, lane, hu[k]);
+                    qk_head_load<HD>(rk + (size_t)kvh * HD, ra.kn, ra.cos_tab, ra.sin_tab, pos, lane, hu[k]);
 #pragma unroll
-                    for (int e = 0; e < E; e++) vv[e] = ra.v[(size_t)kvh * HD + lane + 64 * e];
+                    for (int e = 0; e < E; e++) vv[e] = rv[(size_t)kvh * HD + lane + 64 * e];
                 }
             }
         } else {
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
 #pragma unroll
         for (int k = 0; k < NK; k++) {
             const int e = tid + 256 * k, kr = e / (HD / 4), c = e % (HD / 4);
-            *(float4*)&ks[kr * LD + 4 * c] = kx[k];
+            *(gm_f4*)&ks[kr * LD + 4 * c] = kx[k];
         }
         if (!ROPE) {
 #pragma unroll
@@ -130,8 +133,8 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
 #pragma unroll
                 for (int e = 0; e < E; e++) {
                     ks[(pos - t0) * LD + lane + 64 * e] = o[e];
-                    ra.kc[off + lane + 64 * e] = o[e];
-                    ra.vc[off + lane + 64 * e] = vv[e];
+                    rkc[off + lane + 64 * e] = o[e];
+                    rvc[off + lane + 64 * e] = vv[e];
                 }
             }
         }
@@ -169,6 +172,19 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
     }
 }
 
+template <int HD, int GM, bool ROPE>
+__global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, const float* __restrict__ kc,
+                                                  const int32_t* __restrict__ pos0p, int n_q, int n_kv, int max_seq,
+                                                  float scale, float* __restrict__ S, ScRope ra) {
+    sc1_body<HD, GM, ROPE, false>(q, kc, pos0p, n_q, n_kv, max_seq, scale, S, ra, MsTab{});
+}
+
+template <int HD, int GM>
+__global__ __launch_bounds__(256) void k_attn_sc1_ms(const float* __restrict__ q, const int32_t* __restrict__ pos0p,
+                                                     int n_q, int n_kv, int max_seq, float scale,
+                                                     float* __restrict__ S, ScRope ra, MsTab ms) {
+    sc1_body<HD, GM, true, true>(q, nullptr, pos0p, n_q, n_kv, max_seq, scale, S, ra, ms);
+}
 
 // ---------------------------------------------------------------------------
 // One-token decode over long contexts: the softmax once per score row
@@ -207,6 +223,7 @@ __global__ __launch_bounds__(256) void k_attn_sc1(const float* __restrict__ q, c
 struct SmxWarm {
     const uint8_t* base;
     int rb, n_kv, n_rows;
+    size_t sc_ld;  // score rows of session blockIdx.y start sc_ld apart
 };
 
 DEV void smx_warm(const SmxWarm& W, int L, int max_seq) {
@@ -232,10 +249,9 @@ DEV void smx_warm(const SmxWarm& W, int L, int max_seq) {
     asm volatile("" ::"v"(acc));  // the loaded values count as used: the reads stay
 }
 
-// blockIdx.y: the session (score rows sc_ld apart).
 template <int SEG>
 __global__ __launch_bounds__(SMX_NT) void k_attn_smx(float* __restrict__ S, const int32_t* __restrict__ pos0p,
-                                                  int max_seq, SmxWarm W, size_t sc_ld) {
+                                                  int max_seq, SmxWarm W) {
     constexpr int LDT = 8 * SEG + 4;  // row stride of the transposed copy
     __shared__ __align__(16) float tr[8][LDT];
     __shared__ float tail[8];
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(SMX_NT) void k_attn_smx(float* __restrict__ S, cons
         smx_warm(W, L, max_seq);
         return;
     }
-    float* row = S + blockIdx.y * sc_ld + (size_t)blockIdx.x * max_seq;
+    float* row = S + blockIdx.y * W.sc_ld + (size_t)blockIdx.x * max_seq;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     // zero the positions past the row that the chains read
     for (int i = tid; i < 8 * LDT; i += SMX_NT) (&tr[0][0])[i] = 0.0f;
@@ -766,7 +782,7 @@ __global__ __launch_bounds__(192) void k_attn_pvd(const float* __restrict__ P, c
 // bytes per row) into the L2 that reads them.
 static void smx_launch(void* s, int seg, float* scores, const int32_t* pos0p, int max_seq, int n_q, int n_kv, int G,
                        const void* vbase, int rb, int n_ses = 1, size_t sc_ld = 0) {
-    SmxWarm W{nullptr, rb, n_kv, n_q};
+    SmxWarm W{nullptr, rb, n_kv, n_q, sc_ld};
     int nwarm = 0;
     if (PVD_SMX_WARM && (G == 2 || G == 4) && n_kv % 8 == 0 && vbase) {
         nwarm = (dpuf_hip_cu_count() - n_q) & ~7;
@@ -775,7 +791,7 @@ static void smx_launch(void* s, int seg, float* scores, const int32_t* pos0p, in
     }
     const dim3 g(n_q + nwarm, n_ses);
 #define SMX_CASE(SG) \
-    if (seg == SG) hipLaunchKernelGGL(k_attn_smx<SG>, g, dim3(SMX_NT), 0, ST(s), scores, pos0p, max_seq, W, sc_ld);
+    if (seg == SG) hipLaunchKernelGGL(k_attn_smx<SG>, g, dim3(SMX_NT), 0, ST(s), scores, pos0p, max_seq, W);
     SMX_CASE(16) SMX_CASE(32) SMX_CASE(48) SMX_CASE(64) SMX_CASE(80) SMX_CASE(96) SMX_CASE(128)
 #undef SMX_CASE
 }
@@ -841,11 +857,11 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
         const dim3 g1s(n_kv, (lmax + AS_KC - 1) / AS_KC);                                                         \
         const size_t l1s = (size_t)(AS_KC * (HDV + 8) + GMV * HDV) * 4;                                           \
         if (rope)                                                                                                 \
-            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, true, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q, n_kv, \
-                               max_seq, scale, scores, *rope, MsTab{});                                                    \
+            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, true>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q, n_kv, \
+                               max_seq, scale, scores, *rope);                                                    \
         else                                                                                                      \
-            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, false, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q,      \
-                               n_kv, max_seq, scale, scores, ScRope{}, MsTab{});                                           \
+            hipLaunchKernelGGL((k_attn_sc1<HDV, GMV, false>), g1s, dim3(256), l1s, ST(s), q, kc, pos0p, n_q,      \
+                               n_kv, max_seq, scale, scores, ScRope{});                                           \
     }
 #define WIDE_LAUNCH(HDV)                                                                                          \
     if (gm == 2) SC1_LAUNCH(HDV, 2) else if (gm == 4) SC1_LAUNCH(HDV, 4) else SC1_LAUNCH(HDV, 8)                  \
@@ -894,8 +910,8 @@ int32_t attn_wide_sessions(void* s, int32_t n, int32_t lmax, float* q, const flo
 #define MS_LAUNCH(HDV, GV)                                                                                         \
     {                                                                                                              \
         const size_t l1 = (size_t)(AS_KC * (HDV + 8) + GV * HDV) * 4;                                              \
-        hipLaunchKernelGGL((k_attn_sc1<HDV, GV, true, true>), g1, dim3(256), l1, ST(s), q, NULL, pos, n_q, n_kv,   \
-                           max_seq, scale, scores, r, ms);                                                         \
+        hipLaunchKernelGGL((k_attn_sc1_ms<HDV, GV>), g1, dim3(256), l1, ST(s), q, pos, n_q, n_kv, max_seq, scale,  \
+                           scores, r, ms);                                                                         \
         smx_launch(s, seg, scores, pos, max_seq, n_q, n_kv, G, nullptr, 0, n, ms.sc_ld);                           \
         hipLaunchKernelGGL((k_attn_pvd<HDV, GV, false, true>), dim3(n_kv, HDV * GV / 64, n), dim3(192), 0, ST(s),  \
                            scores, NULL, pos, n_kv, max_seq, out, DpufKvQ8{}, DpufWarm{}, ms);                     \

@@ -942,7 +942,7 @@ static_assert(SK_P % 2 == 0, "the D buffers alternate with the round");
 #define SK_NB 4   // k_gemm_sk round buffers in LDS (producers run up to SK_NB rounds ahead of the chains)
 #endif
 
-#define SKP_P 8  // ring depth in rounds: a multiple of every NR
+#define SKP_P 8  // ring depth in rounds: a multiple of every NR (4 in one instance)
 #define SKP_RB 4                 // blocks per producer wave per round
 #define SKP_RS (SK_NP * SKP_RB)  // 32 blocks per round
 
@@ -1257,7 +1257,8 @@ template <int NR, int MODE>
 __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
     constexpr bool ASYM = MODE != 12;
     constexpr int ND = ASYM ? SKP_RS / 2 : SKP_RS;  // tiles handed over per round
-    static_assert(SKP_P % NR == 0 && NR <= 4, "ring depth must be a multiple of the rounds per fragment");
+    constexpr int P = MODE == 14 && NR == 4 ? 4 : SKP_P;  // mode 14: its high bits would not fit 8 rounds in registers
+    static_assert(P % NR == 0 && NR <= 4, "ring depth must be a multiple of the rounds per fragment");
     __shared__ __align__(16) float dq[2][ND][4][64];        // D (fd of a pair) tiles [buf][block][v][lane]
     __shared__ __align__(16) uint16_t wsl[2][16][SKP_RS];   // weight scales [buf][row][block]
     __shared__ __align__(16) float xsl[2][16][ND + 4];      // token scales (xm_s of a pair) [buf][token][block], rows padded
@@ -1301,8 +1302,8 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
         const int sj = (l >> 2) & 3, sd = l & 3;
         const bool os_hi = ((l >> 4) & 1) != 0;
         const uint32_t oh = (uint32_t)n_blk * 144u + (i16 & 7) * 8;  // mode 14: the row's 8 bytes of high bits
-        uint32_t wq[SKP_P][4], wsq[SKP_P];
-        uint32_t hq[SKP_P][2];
+        uint32_t wq[P][4], wsq[P];
+        uint32_t hq[P][2];
         gm_u4 ax[NR][SKP_RB];
         // token l & 15, per round: mode 12 block l >> 4 of the wave's scale in
         // [0], else the wave's 4 blocks' scales and sums
@@ -1355,14 +1356,14 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
             }
         };
 #pragma unroll
-        for (int u = 0; u < SKP_P - 1; u++) wload(u / NR, u % NR, u);
-        for (int it0 = 0; it0 <= S; it0 += SKP_P) {
+        for (int u = 0; u < P - 1; u++) wload(u / NR, u % NR, u);
+        for (int it0 = 0; it0 <= S; it0 += P) {
 #pragma unroll
-            for (int u = 0; u < SKP_P; u++) {
+            for (int u = 0; u < P; u++) {
                 const int it = it0 + u;
                 if (it > S) break;  // uniform
-                const int un = (u + SKP_P - 1) % SKP_P;
-                wload((it0 + u + SKP_P - 1) / NR, un % NR, un);
+                const int un = (u + P - 1) % P;
+                wload((it0 + u + P - 1) / NR, un % NR, un);
                 const int r = u % NR;
                 if (it < S && r * SKP_RS < n_blk) {
                     const int buf = u & 1;
@@ -1407,15 +1408,15 @@ __global__ __launch_bounds__(64 * (SK_NP + SK_NC)) void k_gemm_skp(GmArgs A) {
     // ---- chain wave c: output (token l % 16, row 4 (l / 16) + c) ----
     const int c = w - SK_NP, rr = 4 * kc + c;
     float acc = 0.0f;
-    for (int it0 = 0; it0 <= S; it0 += SKP_P) {
+    for (int it0 = 0; it0 <= S; it0 += P) {
 #pragma unroll
-        for (int u = 0; u < SKP_P; u++) {
+        for (int u = 0; u < P; u++) {
             const int it = it0 + u;
             if (it > S) break;  // uniform
             if (it >= 1) {
                 // step it - 1: round r of local fragment fl
-                const int um = (u + SKP_P - 1) % SKP_P, r = um % NR;
-                const int fl = (u >= 1 ? it0 : it0 - SKP_P) / NR + um / NR;
+                const int um = (u + P - 1) % P, r = um % NR;
+                const int fl = (u >= 1 ? it0 : it0 - P) / NR + um / NR;
                 const int buf = (u + 1) & 1, b0 = r * SKP_RS;
                 const int nj = min(SKP_RS, n_blk - b0);  // uniform, <= 0 past the last round
                 if (nj > 0) {
