@@ -37,10 +37,12 @@
 //   * A = 16 (u - 8), one v_bitop3 per 4 nibbles (the nibble's top bit
 //     flipped, in a byte's upper half), 3 instructions per nibble word where
 //     u - 8 as fp16 took 11;
-//   * the MFMA's C is the bit pattern 0x3e22f983 (1 / (2 pi)) in every
-//     element: |16 (D - sum8)| < 2^20 stays inside that binade, so the result
-//     read as a float is 1 / (2 pi) + n 2^-26 exactly and one exact
-//     subtraction gives n 2^-26 at full rate (v_cvt_f32_i32 issues at half);
+//   * the MFMA's C is the bit pattern of a float in every element (gm_base: 1.5
+//     2^19, whose last mantissa bit is worth 1 / 16; modes 13 / 14, whose u
+//     needs no offset and no factor, 1.5 2^23, whose last bit is worth 1).
+//     Sums of magnitude up to 2^19 stay inside that binade, so the result read
+//     as a float is the base plus the dot exactly, and one exact subtraction
+//     gives the dot at full rate (v_cvt_f32_i32 issues at half);
 //   * mode 12's products ws * xs come from 4 x 4 outer-product MFMAs (one for
 //     256 outputs in place of 4 v_mul_f32; gm_outer4), issued with the dots
 //     before any result is read: the chains are left with one subtraction and
@@ -49,9 +51,8 @@
 //     waits for each product in turn, they gained nothing.)
 //   * weight scales are widened to float once per workgroup when they are
 //     staged (v_fma_mix_f32 issues at half rate).
-// acc carries the factor 2^-22 (modes 13 / 14, whose u needs no offset:
-// 2^-26), removed at the end: powers of two commute with every rounding here
-// as long as no partial sum is below 2^-104 in magnitude.
+// Dots, products and chains have the reference's own values, so they overflow
+// where its do.
 //
 // Activations (int8, token scales) and weight scales are staged in LDS a
 // stage of several blocks at a time, double-buffered, one barrier per stage.
@@ -140,6 +141,17 @@ DEV gm_f4 gm_outer4(float a, float b) {
     return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, (gm_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
 
+// The float whose bit pattern the dots accumulate onto, and the dot from the
+// accumulated pattern.  (With the base in a scalar register in place of the
+// subtraction's literal, prefill of 512 tokens was 0.9 % slower.)
+template <int MODE>
+constexpr float gm_base = MODE == 12 ? 0x1.8p19f : 0x1.8p23f;
+
+template <int MODE>
+DEV float gm_dot(int d) {
+    return __builtin_bit_cast(float, d) - gm_base<MODE>;
+}
+
 // k_gemm_mfma: NW waves of 16 rows each, TT 16-token tiles per workgroup, for
 // launches with few tiles: a wave of one tile (TT = 1) leaves the most waves,
 // and a tile's serial chain over K is then all of the launch's length.
@@ -155,7 +167,6 @@ k_gemm_mfma(GmArgs A) {
     constexpr int G = TT == 1 ? 4 : TT == 2 ? 2 : 1;  // blocks per LDS read set
     constexpr int NX = NT * SB;              // token scales per stage (512)
     constexpr bool ASYM = MODE != 12;
-    constexpr uint32_t BASE = 0x3e22f983u;   // 1 / (2 pi)
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
     static_assert((2 * QS) % PF == 0, "ring slots are static over two stages");
     static_assert(!SWI || (NW == 8 && MODE == 12), "the SwiGLU pairing: 4 + 4 waves");
@@ -299,7 +310,7 @@ k_gemm_mfma(GmArgs A) {
                 bs[buf][t][2 * p] = ss[k][0];
                 bs[buf][t][2 * p + 1] = ss[k][1];
                 const float pa = (float)sm[k][0] * ss[k][0], pb = (float)sm[k][1] * ss[k][1];
-                bm[ASYM ? buf : 0][t][p] = (pa + pb) * 0.125f * 0x1p-26f;
+                bm[ASYM ? buf : 0][t][p] = (pa + pb) * 0.125f;
             } else {
                 bs[buf][i / SB][i % SB] = ss[k][0];
             }
@@ -322,7 +333,8 @@ k_gemm_mfma(GmArgs A) {
     // scales (and xm_s) of a quad are read with its first set
     long bf[2][G][TT];
     float wsr[2][G][ASYM ? 4 : 1];
-    gm_i4 c0 = {(int)BASE, (int)BASE, (int)BASE, (int)BASE};
+    constexpr int BASE = __builtin_bit_cast(int, gm_base<MODE>);
+    gm_i4 c0 = {BASE, BASE, BASE, BASE};
     asm("" : "+v"(c0));  // loop-invariant registers
     float xs[2][TT][4];
     float xm[2][TT][2];
@@ -422,8 +434,7 @@ k_gemm_mfma(GmArgs A) {
                     float d[4];
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
-                        const int di_v = di[g][t][v];
-                        d[v] = __builtin_bit_cast(float, di_v) - __builtin_bit_cast(float, BASE);
+                        d[v] = gm_dot<MODE>(di[g][t][v]);
                     }
                     if (!ASYM) {
 #pragma unroll
@@ -472,11 +483,6 @@ k_gemm_mfma(GmArgs A) {
             __syncthreads();
         }
     }
-#pragma unroll
-    for (int t = 0; t < TT; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[t][v] *= ASYM ? 0x1p26f : 0x1p22f;
-
     if constexpr (SWI) {
         // SwiGLU + prep of the down input for the workgroup's 64 columns
         // (one 64-block, blk) of the M tokens m0 .. m0 + 63.  Lane l of wave
@@ -558,7 +564,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
     constexpr int PS = SB / 2;               // block pairs per stage
     constexpr int GPW = 8 * RF;              // 8-row groups per workgroup
     constexpr bool ASYM = MODE != 12;
-    constexpr uint32_t BASE = 0x3e22f983u;   // 1 / (2 pi), an inline constant
     static_assert(!SWI || (RF == 2 && MODE == 12), "fragment 0 gate, fragment 1 up");
     __shared__ __align__(16) uint8_t aq[2][SB][NT * 32 + 32];  // int8 activations [stage][block][token][k]
     __shared__ __align__(16) float xl[2][SB][NT + 8];        // token scales
@@ -685,7 +690,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
             xl[buf][2 * p][t] = ss[0];
             xl[buf][2 * p + 1][t] = ss[1];
             const float pa = (float)sm[0] * ss[0], pb = (float)sm[1] * ss[1];
-            ml[ASYM ? buf : 0][p][t] = (pa + pb) * 0.125f * 0x1p-26f;
+            ml[ASYM ? buf : 0][p][t] = (pa + pb) * 0.125f;
         } else {
 #pragma unroll
             for (int k = 0; k < SPT; k++) {
@@ -737,7 +742,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
     float xk[16];
     gm_i16 c0;  // loop-invariant, so that the MFMAs share one set of registers
 #pragma unroll
-    for (int v = 0; v < 16; v++) c0[v] = (int)BASE;
+    for (int v = 0; v < 16; v++) c0[v] = __builtin_bit_cast(int, gm_base<MODE>);
     asm("" : "+v"(c0));
     // block pair p of a stage (blocks 2 p, 2 p + 1; nb of them in range)
     auto pair = [&](int s, int buf, int p, int nb, bool more) {
@@ -800,23 +805,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
                 if (!ASYM) {
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int di = d[f][v];
-                        const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        const float x = gm_dot<MODE>(d[f][v]);
                         acc[f][v] = fmaf(x, pr[f][v >> 2][v & 3], acc[f][v]);
                     }
                 } else if (b == 0) {
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int di = d[f][v];
-                        dk[f][v] = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        dk[f][v] = gm_dot<MODE>(d[f][v]);
                         xk[v] = xs[0][ASYM ? v : 0];
                     }
                     dd[f] = ws[0][f];
                 } else {
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int di = d[f][v];
-                        const float x = __builtin_bit_cast(float, di) - __builtin_bit_cast(float, BASE);
+                        const float x = gm_dot<MODE>(d[f][v]);
                         const float p1 = x * xs[1][ASYM ? v : 0];
                         const float fd = fmaf(dk[f][v], xk[v], p1);
                         acc[f][v] = fmaf(fd, dd[f], acc[f][v]);
@@ -860,11 +862,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RF == 1 && 
             __syncthreads();
         }
     }
-    const float rescale = ASYM ? 0x1p26f : 0x1p22f;
-#pragma unroll
-    for (int f = 0; f < RF; f++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[f][v] *= rescale;
 
     if constexpr (SWI) {
         constexpr int XS = 68;

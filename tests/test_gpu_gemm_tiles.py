@@ -47,3 +47,35 @@ def test_gemm_tiles(eng, orc, mode, cols, rows, m):
                                 d.sign_bits, M.ptr(out_o))
     assert np.isfinite(out_o).all()
     assert bits_equal(out_g, out_o), maxdiff(out_g, out_o)
+
+
+@pytest.mark.parametrize("mode", [12, 13, 14])
+@pytest.mark.parametrize("rows,m", [(40, 5), (4136, 12)] + SIZES)
+def test_gemm_overflow(eng, orc, mode, rows, m):
+    """Inputs whose partial sums pass the largest float: an output is infinite
+    exactly where the reference's chain is (its infinities never come back into
+    range, also where the full sum would), in every kernel above one token.
+    The spread of a chain's end is 113 sqrt(blocks) times that of the inputs (32
+    products with weights of 20 a block): a good part of the largest float, in
+    modes 13 and 14 less, whose unsigned dots pass through larger sums."""
+    cols = 192 if rows * m > 5e6 else 320
+    W = M.random_normal(rows * cols, 20.0, 17 + mode, f"o{rows}x{cols}").reshape(rows, cols)
+    blob, d = M.pack_matrix(W, M.sign_bits(cols, 7, f"os{rows}x{cols}"), mode=mode)
+    sd = (0.7 if mode == 12 else 0.35) * 3.4e38 / (113 * np.sqrt(cols / 32))
+    x = (np.random.default_rng(rows + cols + m).standard_normal((m, cols)) * sd).astype(np.float32)
+    out_g = np.full((m, rows), np.nan, np.float32)
+    out_o = np.full((m, rows), np.nan, np.float32)
+    log(f"overflow: mode {mode} rows={rows} cols={cols} M={m}")
+    getattr(eng, f"dpuf_matmul_qr_{NAMES[mode]}_f32")(m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base,
+                                                      d.tile_offsets, d.sign_bits, M.ptr(out_g))
+    if mode == 12:
+        orc.orc_matmul_f32(m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base, d.tile_offsets, d.sign_bits,
+                           M.ptr(out_o))
+    else:
+        orc.orc_matmul_asym_f32(int(mode == 14), m, rows, cols, d.n_tiles, M.ptr(x), d.tensor_base, d.tile_offsets,
+                                d.sign_bits, M.ptr(out_o))
+    bad = ~np.isfinite(out_o)
+    assert 0.01 < bad.mean() < 0.99, bad.mean()
+    nan = np.isnan(out_o)
+    assert np.array_equal(np.isnan(out_g), nan)
+    assert bits_equal(np.where(nan, 0, out_g), np.where(nan, 0, out_o)), (~np.isfinite(out_g)).sum() - bad.sum()
