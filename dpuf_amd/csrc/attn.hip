@@ -850,11 +850,11 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     const int qt1 = 32 / G < M ? 32 / G : M;
     const dim3 g1(n_kv, (M + qt1 - 1) / qt1, (lmax + AS_KC - 1) / AS_KC);
     const size_t lds1 = (size_t)(AS_KC + 32) * (hd + 4) * 4;
-    const size_t budget = 112 * 1024;  // LDS bytes of a workgroup's probability rows
-    // several tokens, an even group of up to 16: the matrix-instruction
-    // kernels.  Less than one 16-row tile (M G < 16) over keys whose rows
-    // exceed the split kernels' LDS budget stays on the one-pair kernel.
-    if (M > 1 && (M * G >= 16 || (size_t)G * ((lmax + 7) & ~7) * 4 <= budget)) {
+    // several tokens, an even group of up to 16: the matrix-instruction kernels,
+    // at any length (2 tokens, groups of 4, 4 layers of 8 KV heads at 7 300
+    // keys: 1.03 ms a call against 9.2 on the one-pair kernel, at 18 000 keys
+    // 2.3 against 29.7)
+    if (M > 1) {
         DpufPrep fop = op;
         if (!prepped) fop.q = NULL;
         if (attn_tile(s, M, lmax, q, kc, vc, NULL, out, scores, pos0p, n_q, n_kv, hd, max_seq, scale, o_sign, fop) ==
@@ -874,6 +874,7 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     // rows per workgroup keeps >= 32 dims per P.V chain group, so the
     // softmax each dim chunk repeats stays small next to P.V
     const int lcap = (lmax + 7) & ~7;
+    const size_t budget = 112 * 1024;
     int qt2 = 8 / G > 1 ? 8 / G : 1;
     if (qt2 > M) qt2 = M;
     while (qt2 > 1 && (size_t)qt2 * G * lcap * 4 > budget) qt2--;

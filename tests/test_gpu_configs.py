@@ -297,26 +297,35 @@ def test_graph_bucket_with_large_max_seq(eng, orc):
     p.close()
 
 
-def test_attention_beyond_split_lds_budget(eng, orc):
-    """Groups of 4 with 7200 cached positions.  A two-token forward there:
-    its rows of probabilities no longer fit the split kernels' LDS budget, so
-    it takes the one-pair-per-workgroup kernel (k_attn); then one-token decode
-    steps (the three-launch long-context path).  Logits bit-identical."""
-    shape = dict(hidden_size=256, intermediate_size=512, num_layers=1, num_q_heads=8, num_kv_heads=2,
-                 head_dim=128, vocab_size=4096, tie_word_embeddings=1)
-    m = M.Model.build(shape, max_seq_len=7240, seed=81)
+TILES = 0  # dpuf_amd_attn_path_count: the matrix-instruction kernels of several tokens
+
+
+@pytest.mark.parametrize("nq,hd,ctx,path", [(8, 128, 7200, TILES), (36, 64, 1700, FALLBACK)])
+def test_attention_beyond_split_lds_budget(eng, orc, nq, hd, ctx, path):
+    """A two-token forward whose rows of probabilities no longer fit the split
+    kernels' LDS budget.  Groups of 4 with 7 200 cached positions: the
+    matrix-instruction kernels.  Groups of 18 with 1 700, which those do not
+    serve: the one-pair-per-workgroup kernel (k_attn).  Then one-token decode
+    steps (groups of 4: the three-launch long-context path).  Logits
+    bit-identical."""
+    shape = dict(hidden_size=256, intermediate_size=512, num_layers=1, num_q_heads=nq, num_kv_heads=2,
+                 head_dim=hd, vocab_size=4096, tie_word_embeddings=1)
+    m = M.Model.build(shape, max_seq_len=ctx + 40, seed=81)
     p = Pair(eng, orc, m)
     rng = np.random.default_rng(82)
     for kvh in range(2):
-        p.set_kv(0, kvh, 0, rng.standard_normal((7200, 128), dtype=np.float32),
-                 rng.standard_normal((7200, 128), dtype=np.float32))
-    log("k_attn fallback: two tokens at position 7200")
-    f0 = eng.dpuf_amd_attn_path_count(FALLBACK)
-    lg, lo = p.forward(np.array([3, 4000], np.int32), 7200, only_last=0)
+        p.set_kv(0, kvh, 0, rng.standard_normal((ctx, hd), dtype=np.float32),
+                 rng.standard_normal((ctx, hd), dtype=np.float32))
+    log(f"two tokens at position {ctx}, groups of {nq // 2}")
+    c0, f0 = eng.dpuf_amd_attn_path_count(path), eng.dpuf_amd_attn_path_count(FALLBACK)
+    lg, lo = p.forward(np.array([3, 4000], np.int32), ctx, only_last=0)
     assert bits_equal(lg, lo), maxdiff(lg, lo)
-    assert eng.dpuf_amd_attn_path_count(FALLBACK) - f0 == 1
-    greedy(p, lg, lo, 7202, 3, "after fallback")
-    assert eng.dpuf_amd_attn_path_count(FALLBACK) - f0 == 1  # the one-token steps take the wide kernels
+    assert eng.dpuf_amd_attn_path_count(path) - c0 == 1
+    f1 = eng.dpuf_amd_attn_path_count(FALLBACK)
+    assert f1 - f0 == (path == FALLBACK)
+    greedy(p, lg, lo, ctx + 2, 3, "after two tokens")
+    if path == TILES:
+        assert eng.dpuf_amd_attn_path_count(FALLBACK) == f1  # the one-token steps take the wide kernels
     p.close()
 
 
