@@ -1025,6 +1025,7 @@ void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8
                        n_q, n_kv, hd, max_seq);
     LAUNCHED("k_attn_q8_sc/k_attn_q8");
     attn_path_note(5);
+    attn_path_note(7);
 }
 
 void dpuf_hip_q8_rows(void* s, const float* k, const float* v, int32_t n, int32_t hd, DpufKvQ8 c8, size_t row0) {

@@ -655,9 +655,11 @@ static void launch(void* s, int M, int lmax, const float* q, const float* kc, co
     if (res <= 76 * 1024)  // two workgroups per CU at least
         hipLaunchKernelGGL((k_attn_pvm<HD, Q8, true>), g2, dim3(2 * HD), res, ST(s), S, smax, vc, c8, pos0, M, n_q,
                            n_kv, max_seq, qp, (int)tpw, out, o_sign, op);
-    else
+    else {
         hipLaunchKernelGGL((k_attn_pvm<HD, Q8, false>), g2, dim3(2 * HD), P::lds(2), ST(s), S, smax, vc, c8, pos0, M,
                            n_q, n_kv, max_seq, qp, (int)tpw, out, o_sign, op);
+        attn_path_note(6);
+    }
 }
 
 int32_t attn_tile(void* s, int32_t M, int32_t lmax, const float* q, const float* kc, const float* vc,

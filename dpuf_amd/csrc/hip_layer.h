@@ -262,7 +262,7 @@ int32_t dpuf_hip_attn_sessions(void* s, int32_t n, int32_t lmax, float* q, const
                                float scale);
 /* Attention launches enqueued per path (dpuf_amd_attn_path_count); -1 for
  * another `which`. */
-#define DPUF_HIP_ATTN_PATHS 6
+#define DPUF_HIP_ATTN_PATHS 8
 int64_t dpuf_hip_attn_path_count(int32_t which);
 void dpuf_hip_zero_rows(void* s, int32_t M, float* out, int32_t ld, int32_t r0, int32_t r1);
 /* CRC32 of n tile bodies (base + off[t], len[t] bytes) against want[t]: ok[t] = 1 when equal. */

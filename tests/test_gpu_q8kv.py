@@ -124,22 +124,29 @@ def test_q8_prefix_slots_and_refusals(eng, orc):
     p.close()
 
 
-def test_q8_rows_beyond_lds(eng, orc):
-    """7200 cached positions with groups of 4: a two-token forward's
-    probability rows no longer fit the split kernel's LDS budget, so it takes
-    the softmax-in-memory kernel (k_attn_q8); one-token steps after it take
-    the split kernel again.  Bit-identical."""
-    shape = dict(TINY, num_layers=1, num_q_heads=8, num_kv_heads=2, head_dim=128)
-    m, cfg = q8_model(shape, 7240, 231)
+Q8_MEMORY = 7  # dpuf_amd_attn_path_count: the int8 softmax-in-memory kernel
+
+
+@pytest.mark.parametrize("nq,hd,ctx,memory", [(8, 128, 7200, 0), (36, 64, 1700, 1)])
+def test_q8_rows_beyond_lds(eng, orc, nq, hd, ctx, memory):
+    """Probability rows past the split kernel's LDS budget.  Groups of 4 at
+    7 200 positions: a two-token forward takes the matrix-instruction kernels,
+    which stream them.  Groups of 18 at 1 700, which those do not serve: the
+    softmax-in-memory kernel (k_attn_q8).  One-token steps after each.
+    Bit-identical."""
+    shape = dict(TINY, num_layers=1, num_q_heads=nq, num_kv_heads=2, head_dim=hd)
+    m, cfg = q8_model(shape, ctx + 40, 231)
     p = Q8Pair(eng, orc, m, cfg)
     rng = np.random.default_rng(232)
     for kvh in range(2):
-        p.set_kv(0, kvh, 0, rng.standard_normal((7200, 128), dtype=np.float32),
-                 rng.standard_normal((7200, 128), dtype=np.float32))
-    log("q8 kv: two tokens at position 7200")
-    lg, lo = p.forward(np.array([3, 4000], np.int32), 7200, only_last=0)
+        p.set_kv(0, kvh, 0, rng.standard_normal((ctx, hd), dtype=np.float32),
+                 rng.standard_normal((ctx, hd), dtype=np.float32))
+    log(f"q8 kv: two tokens at position {ctx}, groups of {nq // 2}")
+    m0 = eng.dpuf_amd_attn_path_count(Q8_MEMORY)
+    lg, lo = p.forward(np.array([3, 4000], np.int32), ctx, only_last=0)
+    assert eng.dpuf_amd_attn_path_count(Q8_MEMORY) - m0 == memory
     assert bits_equal(lg, lo), maxdiff(lg, lo)
-    greedy(p, lg, lo, 7202, 3, "q8 after 7200")
+    greedy(p, lg, lo, ctx + 2, 3, f"q8 after {ctx}")
     p.close()
 
 
