@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from dpuf_amd import model as M
-from test_gpu_configs import bits_equal, log, maxdiff
+from test_gpu_configs import Pair, bits_equal, log, maxdiff
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +79,21 @@ def test_gemm_overflow(eng, orc, mode, rows, m):
     nan = np.isnan(out_o)
     assert np.array_equal(np.isnan(out_g), nan)
     assert bits_equal(np.where(nan, 0, out_g), np.where(nan, 0, out_o)), (~np.isfinite(out_g)).sum() - bad.sum()
+
+
+@pytest.mark.parametrize("n", [17, 29, 31, 32, 33, 70])
+def test_gate_up_swiglu_tiles(eng, orc, n):
+    """Gate, up, SwiGLU and the down input's prep in one launch (16 384 gate +
+    up rows or more): tokens that fill its tile or end inside it, and 129
+    64-column blocks, one past a multiple of the 8 XCDs.  Every row's residual
+    of each layer and its logits."""
+    shape = dict(hidden_size=256, intermediate_size=8256, num_layers=2, num_q_heads=4, num_kv_heads=2, head_dim=64,
+                 vocab_size=512, tie_word_embeddings=1)
+    p = Pair(eng, orc, M.Model.build(shape, max_seq_len=96, seed=411))
+    p.capture(n)
+    log(f"gate + up + SwiGLU: {n} tokens, 8 256 columns")
+    lg, lo = p.forward(np.random.default_rng(412 + n).integers(0, 512, n).astype(np.int32), 0, only_last=0)
+    cg, co = p.captured(n)
+    assert bits_equal(cg, co), maxdiff(cg, co)
+    assert bits_equal(lg, lo), maxdiff(lg, lo)
+    p.close()
