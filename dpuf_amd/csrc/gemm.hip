@@ -89,7 +89,7 @@ struct GmJob {
 struct GmArgs {
     GmJob j[3];
     int n_jobs;
-    int tb[4];  // prefix sums of 16-group row tiles per job
+    int tb[4];  // prefix sums of the jobs' row tiles (workgroups or fragments of the kernel)
     int K, M;
     int gy;     // token tiles
     // rows [z0, z1) of zo (row stride zld) set to 0 by zt extra row tiles of
@@ -97,7 +97,7 @@ struct GmArgs {
     float* zo;
     int zld, z0, z1, zt;
     int32_t* err;  // device error word: set when a bounded wait of k_gemm_sk runs out
-    // gate + up with the SwiGLU (k_gemm_mfma<..., true>): the prep of the
+    // gate + up with the SwiGLU (the SWI instances): the prep of the
     // down projection's input [M][swI] goes to swo, with the down input's
     // sign bits swsign and dead zone swdz
     DpufPrep swo;
@@ -156,7 +156,7 @@ DEV float gm_dot(int d) {
 // launches with few tiles: a wave of one tile (TT = 1) leaves the most waves,
 // and a tile's serial chain over K is then all of the launch's length.
 template <int TT, int MODE, int NW, bool SWI>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : TT == 1 || (MODE != 12 && TT == 4) ? 2 : 3))) void
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : TT == 1 ? 2 : 3))) void
 k_gemm_mfma(GmArgs A) {
     constexpr int NT = 16 * TT;              // tokens per workgroup
     constexpr int NTH = 64 * NW;             // threads per workgroup
@@ -164,10 +164,10 @@ k_gemm_mfma(GmArgs A) {
     constexpr int SB = 32 / TT;              // blocks per LDS stage
     constexpr int QS = SB / 4;               // 4-block quads per stage
     constexpr int PF = TT == 1 ? 8 : 4;      // quads of nibbles in flight
-    constexpr int G = TT == 1 ? 4 : TT == 2 ? 2 : 1;  // blocks per LDS read set
+    constexpr int G = TT == 1 ? 4 : 2;       // blocks per LDS read set
     constexpr int NX = NT * SB;              // token scales per stage (512)
     constexpr bool ASYM = MODE != 12;
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
+    static_assert((NW == 4 || NW == 8) && (TT == 1 || TT == 2), "4 or 8 waves, 16 or 32 tokens");
     static_assert((2 * QS) % PF == 0, "ring slots are static over two stages");
     static_assert(!SWI || (NW == 8 && MODE == 12), "the SwiGLU pairing: 4 + 4 waves");
     __shared__ __align__(16) uint8_t bq[2][SB][NT * 32 + 32];          // int8 activations [stage][block][token][k]
@@ -485,7 +485,7 @@ k_gemm_mfma(GmArgs A) {
     }
     if constexpr (SWI) {
         // SwiGLU + prep of the down input for the workgroup's 64 columns
-        // (one 64-block, blk) of the M tokens m0 .. m0 + 63.  Lane l of wave
+        // (one 64-block, blk) of the tokens m0 .. m0 + NT - 1 below M.  Lane l of wave
         // w holds acc[t][v] for column c = 16 (w & 3) + 4 (l / 16) + v and
         // token 16 t + l % 16; x[w & 3][t][v][l] in the LDS of the stage
         // buffers (free once every wave is past its last block) exchanges
@@ -1514,7 +1514,7 @@ int32_t dpuf_hip_gemm_swiglu(void* s, int32_t M, const DpufGemvJob* jobs, float 
     const int I = a.w.rows;
     if (M <= 16 || a.w.mode != 12 || b.w.mode != 12 || a.w.cols != b.w.cols || b.w.rows != I || I % 64 ||
         2 * I < GM_SWI_ROWS || a.g0 != 0 || b.g0 != 0 || a.g1 != I / 8 || b.g1 != I / 8 || !a.p.q || a.p.q != b.p.q ||
-        a.p.s != b.p.s || !out.q || !out.s || !out.m || !out.h || out.h == a.p.h || out.q == a.p.q)
+        a.p.s != b.p.s || !out.q || !out.s || !out.m || out.q == a.p.q)
         return -1;
     if ((long long)M * a.w.cols >= (1ll << 30) || (long long)M * I >= (1ll << 30)) return -1;
     GmArgs G;
@@ -1528,7 +1528,7 @@ int32_t dpuf_hip_gemm_swiglu(void* s, int32_t M, const DpufGemvJob* jobs, float 
         G.j[i].g1 = jobs[i].g1;
         G.j[i].rows = jobs[i].w.rows;
         G.j[i].h = jobs[i].p.h;
-            G.j[i].q = jobs[i].p.q;
+        G.j[i].q = jobs[i].p.q;
         G.j[i].s = jobs[i].p.s;
         G.j[i].m = jobs[i].p.m;
         G.j[i].out = jobs[i].out;
@@ -1575,8 +1575,13 @@ void dpuf_hip_gm_launch(void* s, int32_t M, int32_t n_jobs, const DpufGemvJob* j
                 note(hipErrorInvalidValue, "dpuf_hip_gemv: M * K must stay below 2^30");
                 return;
             }
-            if (!jobs[i].p.h) {
-                note(hipErrorInvalidValue, "dpuf_hip_gemv: M > 1 needs the fp16 activations (DpufPrep.h)");
+            // the K-split kernels read the fp16 copy, the others the int8 one
+            if (M <= 16 && !jobs[i].p.h) {
+                note(hipErrorInvalidValue, "dpuf_hip_gemv: 2..16 tokens need the fp16 activations (DpufPrep.h)");
+                return;
+            }
+            if (M > 16 && !jobs[i].p.q) {
+                note(hipErrorInvalidValue, "dpuf_hip_gemv: more than 16 tokens need the int8 activations (DpufPrep.q)");
                 return;
             }
             G.j[i].s = jobs[i].p.s;

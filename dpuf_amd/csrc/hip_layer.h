@@ -34,8 +34,8 @@ typedef struct {
 static inline int32_t dpuf_grp_unit(int32_t mode) { return mode == 14 ? 208 : 144; }
 
 /* Prepped activations of M rows: q int8 [M][K], s f32 [M][K/32], m i32 [M][K/32],
- * and h, the same q as fp16 [M][K] (the M > 1 GEMM's input; the prep
- * kernels fill it when non-NULL and M > 1). */
+ * and h, the same q as fp16 [M][K] (the input of the GEMMs of 2..16 tokens, in
+ * place of q; the prep kernels fill it when non-NULL and M > 1). */
 typedef struct {
     int8_t*  q;
     float*   s;

@@ -93,6 +93,40 @@ def test_engine_refuses_to_run_without_hip_device():
     assert not eng.dpuf_engine_create(*m.create_args())
 
 
+class _Prep(C.Structure):
+    _fields_ = [(f, C.c_void_p) for f in "qsmh"]
+
+
+class _Job(C.Structure):  # DpufGemvJob of hip_layer.h
+    _fields_ = [("g", C.c_void_p), ("sign", C.c_void_p), ("rows", C.c_int32), ("cols", C.c_int32),
+                ("n_groups", C.c_int32), ("mode", C.c_int32), ("g0", C.c_int32), ("g1", C.c_int32), ("p", _Prep),
+                ("out", C.c_void_p), ("ldo", C.c_int32)]
+
+
+@pytest.mark.parametrize("m,missing", [(5, "h"), (16, "h"), (17, "q"), (512, "q")])
+@pytest.mark.parametrize("mode", [12, 13, 14])
+def test_gemm_refuses_missing_activations(mode, m, missing):
+    """A GEMM launch without the activations its kernels read (2..16 tokens
+    the fp16 copy, more the int8 values) is refused before anything is
+    launched."""
+    eng = abi.load_engine()
+    if eng.dpuf_amd_device_ok():
+        pytest.skip("a HIP device is visible: the other pointers here are not device memory")
+    L = C.CDLL(eng._name)
+    L.dpuf_hip_gm_launch.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(_Job), C.c_void_p] + [C.c_int32] * 3
+    L.dpuf_hip_gm_launch.restype = None
+    L.dpuf_hip_error_string.restype = C.c_char_p
+    buf = (C.c_char * 64)()
+    at = C.addressof(buf)
+    j = _Job(g=at, rows=64, cols=64, n_groups=8, mode=mode, g0=0, g1=8, out=at, ldo=64,
+             p=_Prep(**{f: None if f == missing else at for f in "qsmh"}))
+    L.dpuf_hip_clear_error()
+    L.dpuf_hip_gm_launch(None, m, 1, C.byref(j), None, 0, 0, 0)
+    assert L.dpuf_hip_ok() == 0
+    assert f"DpufPrep.{missing}" in L.dpuf_hip_error_string().decode()
+    L.dpuf_hip_clear_error()
+
+
 def test_crc32_known_answer(tools):
     data = np.frombuffer(b"123456789", np.uint8).copy()
     assert tools.dpuf_crc32_bytes(M.ptr(data), 9) == 0xCBF43926
