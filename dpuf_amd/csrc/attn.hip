@@ -252,14 +252,14 @@ __global__ __launch_bounds__(AP_NT) void k_attn_pv(const float* __restrict__ S, 
     v_load(0);
     // score rows -> LDS by direct-to-LDS loads (1 KB per wave instruction,
     // all in flight together; the last one may run into the padding);
-    // elements past a row's length are don't-care
+    // elements past a row's length are don't-care (the last piece of a row may
+    // end in the next row, or past the last row in the scratch's maxima)
     {
         const int n4w = lcap >> 2, tot = R * n4w;
         for (int base = wv * 64; base < tot; base += AP_NT) {
             const int e = base + lane, r = e / n4w, c = e % n4w;
             const int rr = e < tot ? r : 0, mq = m0 + rr / G < M ? m0 + rr / G : M - 1;
-            int t = 4 * c;
-            if (e >= tot || t + 3 >= max_seq) t = 0;
+            const int t = e < tot ? 4 * c : 0;
             const float* src = S + ((size_t)mq * n_q + kvh * G + rr % G) * max_seq + t;
             __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr_t)(P + 4 * base), 16, 0, 0);
         }

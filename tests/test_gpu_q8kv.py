@@ -172,6 +172,28 @@ def test_q8_4096_injected_keys(eng, orc, nq):
     p.close()
 
 
+@pytest.mark.parametrize("kv_type", [0, 1])
+@pytest.mark.parametrize("n", [1, 5])
+@pytest.mark.parametrize("nq,max_seq", [(6, 301), (6, 302), (6, 303), (36, 303)])
+def test_odd_groups_last_positions_unaligned_max_seq(eng, orc, nq, max_seq, n, kv_type):
+    """Groups of 3 and 18 (the split kernels) up to the last position of an
+    engine whose max_seq is not a multiple of 4: the last 16-byte piece of a
+    score row runs past it."""
+    shape = dict(TINY, num_layers=1, num_q_heads=nq, num_kv_heads=2, head_dim=64)
+    m, cfg = q8_model(shape, max_seq, 311)
+    cfg.kv_type = kv_type
+    p = Q8Pair(eng, orc, m, cfg)
+    rng = np.random.default_rng(312)
+    ctx = max_seq - n
+    for kvh in range(2):
+        p.set_kv(0, kvh, 0, rng.standard_normal((ctx, 64), dtype=np.float32),
+                 rng.standard_normal((ctx, 64), dtype=np.float32))
+    log(f"max_seq {max_seq}, groups of {nq // 2}, kv_type {kv_type}: the last {n} positions")
+    lg, lo = p.forward(np.arange(n, dtype=np.int32), ctx, only_last=0)
+    assert bits_equal(lg, lo), maxdiff(lg, lo)
+    p.close()
+
+
 @pytest.mark.parametrize("nq,nkv,kv_type", [(8, 2, 0), (4, 2, 0), (16, 2, 0), (8, 2, 1), (4, 2, 1)])
 def test_one_token_last_positions_unaligned_max_seq(eng, orc, nq, nkv, kv_type):
     """An engine created for 1029 positions (not a multiple of 4) decoding its
