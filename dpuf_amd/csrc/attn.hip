@@ -1009,7 +1009,8 @@ void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8
 #define PVQ(HDV, NT)                                                                                              \
     hipLaunchKernelGGL((k_attn_pv<HDV, NT, true>), g2, dim3(NT), lds2, ST(s), scores, nullptr, pos0, M, n_q, n_kv, \
                        max_seq, qt2, dw, lcap, vk, out, c8.vq, c8.vs)
-        if (lds2 <= 160 * 1024) {
+        const size_t own = (size_t)((wide ? 1024 : 256) + 2 * 32) * 4;  // the kernel's own arrays
+        if (lds2 + own <= 160 * 1024) {
             if (hd == 64) { if (wide) PVQ(64, 1024); else PVQ(64, 256); }
             else if (hd == 128) { if (wide) PVQ(128, 1024); else PVQ(128, 256); }
             else { if (wide) PVQ(256, 1024); else PVQ(256, 256); }

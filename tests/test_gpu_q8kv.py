@@ -150,6 +150,24 @@ def test_q8_rows_beyond_lds(eng, orc, nq, hd, ctx, memory):
     p.close()
 
 
+@pytest.mark.parametrize("n,ctx", [(1, 799), (1, 790), (2, 800)])
+def test_q8_rows_that_just_fill_lds(eng, orc, n, ctx):
+    """Groups of 16 at about 800 positions: the split kernel's rows and chunks
+    fit 160 KB of LDS, but not with the kernel's own 4 352 bytes.  Such a step
+    was refused with a launch error; it takes the softmax in memory."""
+    shape = dict(TINY, num_layers=1, num_q_heads=32, num_kv_heads=2, head_dim=64)
+    m, cfg = q8_model(shape, 820, 241)
+    p = Q8Pair(eng, orc, m, cfg)
+    rng = np.random.default_rng(242)
+    for kvh in range(2):
+        p.set_kv(0, kvh, 0, rng.standard_normal((ctx, 64), dtype=np.float32),
+                 rng.standard_normal((ctx, 64), dtype=np.float32))
+    log(f"q8 kv: {n} tokens at position {ctx}, groups of 16")
+    lg, lo = p.forward(np.arange(n, dtype=np.int32), ctx, only_last=0)
+    assert bits_equal(lg, lo), maxdiff(lg, lo)
+    p.close()
+
+
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("nq", [32, 64])
 def test_q8_4096_injected_keys(eng, orc, nq):
