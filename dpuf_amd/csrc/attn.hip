@@ -829,6 +829,61 @@ void dpuf_hip_qk_rope_kv(void* s, int32_t M, float* q, float* k, const float* v,
     LAUNCHED("k_qk_rope_kv");
 }
 
+// Geometry of the split softmax + P.V launch (k_attn_pv): tiles of qt tokens x
+// G heads, the head dim in dc chunks of dw, V chunks of vk keys.  About 8 rows
+// per workgroup keep >= 32 dims per P.V chain group, so the softmax each dim
+// chunk repeats stays small next to P.V; the int8 cache's chunks lie inside
+// one 32-column block.  1024 threads for launches of few workgroups (decode:
+// the softmax phases go 4x wider), 256 when many workgroups already fill the
+// chip (prefill).  fits: the rows of probabilities, the chunks and the kernel's
+// own arrays fit in LDS.
+struct PvSplit {
+    int qt, dc, dw, vk, tiles, threads;
+    size_t lds;
+    bool fits;
+};
+
+static PvSplit pv_split(int M, int lmax, int n_kv, int G, int hd, bool q8) {
+    PvSplit p;
+    const size_t budget = 112 * 1024, lcap = (lmax + 7) & ~7;
+    p.qt = 8 / G > 1 ? 8 / G : 1;
+    if (p.qt > M) p.qt = M;
+    while (p.qt > 1 && p.qt * G * lcap * 4 > budget) p.qt--;
+    const int R = p.qt * G;
+    p.dc = 1;
+    while (p.dc < hd / 4 && R * (hd / p.dc) > 256) p.dc *= 2;
+    p.tiles = n_kv * ((M + p.qt - 1) / p.qt);
+    while (p.dc < hd / 4 && p.tiles * p.dc < 128) p.dc *= 2;  // enough workgroups to spread the V reads
+    while (q8 && hd / p.dc > 32) p.dc *= 2;
+    p.dw = hd / p.dc;
+    p.vk = 4096 / p.dw;  // V chunk: 16 KB (+ padding), two buffers
+    p.lds = (((R * lcap + 1023) & ~(size_t)1023) + 2 * (size_t)(p.vk + 4) * p.dw +
+             (q8 ? 2 * (size_t)p.vk + (size_t)R * p.vk : 0)) * 4;
+    p.threads = (long long)p.tiles * p.dc < 1024 ? 1024 : 256;
+    const size_t own = (size_t)(p.threads + 2 * 32) * 4;  // part, rowv
+    p.fits = G <= 32 && R * lcap * 4 <= budget && (!q8 || p.lds + own <= 160 * 1024);
+    return p;
+}
+
+// Several tokens: whether the split kernels beat the matrix-instruction ones.
+// Those walk all the keys of 16 score rows in one workgroup, whatever the head
+// dim; a few tokens over many keys are a few such workgroups, while the split
+// P.V gives each a fraction of the dims.  So the split kernels win as long as
+// their grid is one workgroup per CU at most, from a length on that grows with
+// what a workgroup repeats or shares.  us per layer, split | tiles, 8 KV heads,
+// groups of 4, head dim 128, fp32: 2 tokens at 300 keys 57 | 55, 600 61 | 62,
+// 1 100 64 | 79, 2 000 74 | 106, 4 000 87 | 162; 16 tokens (256 workgroups) at
+// 4 000 139 | 171, 24 (384) 214 | 178.  int8 cache: 2 tokens at 4 000 98 | 169,
+// 24 at 4 000 287 | 189.  The int8 softmax in memory, where the split kernel's
+// rows do not fit LDS, wins likewise at head dim 64 only (groups of 16, 2
+// tokens at 4 000 163 | 196; head dim 128, groups of 8, 187 | 173).
+static bool split_first(const PvSplit& p, int M, int lmax, int n_kv, int G, int hd, bool q8) {
+    const int n_cu = dpuf_hip_cu_count();
+    if (lmax <= (q8 ? 48 * G + 96 : 3 * hd + 8 * G + 40)) return false;
+    if (p.fits) return p.tiles * p.dc <= n_cu;
+    return q8 && hd == 64 && M * n_kv * ((G + 1) / 2) <= n_cu;
+}
+
 // Split attention (k_attn_sc + k_attn_pv) over keys up to lmax = pos0 + M
 // (or max_seq when the launch is captured for replay at any position).
 // Returns -1 without launching when the shape does not fit (group > 32, head
@@ -850,11 +905,12 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     const int qt1 = 32 / G < M ? 32 / G : M;
     const dim3 g1(n_kv, (M + qt1 - 1) / qt1, (lmax + AS_KC - 1) / AS_KC);
     const size_t lds1 = (size_t)(AS_KC + 32) * (hd + 4) * 4;
-    // several tokens, an even group of up to 16: the matrix-instruction kernels,
-    // at any length (2 tokens, groups of 4, 4 layers of 8 KV heads at 7 300
-    // keys: 1.03 ms a call against 9.2 on the one-pair kernel, at 18 000 keys
-    // 2.3 against 29.7)
-    if (M > 1) {
+    // several tokens, an even group of up to 16: the matrix-instruction kernels
+    // but for the split ones' range; also where the rows fit no LDS (2 tokens,
+    // groups of 4, 4 layers of 8 KV heads at 7 300 keys: 1.03 ms a call against
+    // 9.2 on the one-pair kernel, at 18 000 keys 2.3 against 29.7)
+    const PvSplit pv = pv_split(M, lmax, n_kv, G, hd, false);
+    if (M > 1 && !split_first(pv, M, lmax, n_kv, G, hd, false)) {
         DpufPrep fop = op;
         if (!prepped) fop.q = NULL;
         if (attn_tile(s, M, lmax, q, kc, vc, NULL, out, scores, pos0p, n_q, n_kv, hd, max_seq, scale, o_sign, fop) ==
@@ -870,28 +926,13 @@ static int32_t attn_split(void* s, int32_t M, int32_t lmax, const float* q, cons
     if (M == 1 && attn_wide_f32(s, lmax, q, kc, vc, out, scores, pos0p, n_q, n_kv, hd, max_seq, scale, rope, wm) == 0)
         return 0;
     if (rope) return -1;
-    // softmax + P.V in LDS: R = qt2 * G rows of lcap probabilities; about 8
-    // rows per workgroup keeps >= 32 dims per P.V chain group, so the
-    // softmax each dim chunk repeats stays small next to P.V
-    const int lcap = (lmax + 7) & ~7;
-    const size_t budget = 112 * 1024;
-    int qt2 = 8 / G > 1 ? 8 / G : 1;
-    if (qt2 > M) qt2 = M;
-    while (qt2 > 1 && (size_t)qt2 * G * lcap * 4 > budget) qt2--;
-    if ((size_t)qt2 * G * lcap * 4 > budget) return -1;
-    const int R = qt2 * G;
-    int dc = 1;
-    while (dc < hd / 4 && R * (hd / dc) > 256) dc *= 2;
-    const int tiles = n_kv * ((M + qt2 - 1) / qt2);
-    while (dc < hd / 4 && tiles * dc < 128) dc *= 2;  // enough workgroups to spread the V reads
-    const int dw = hd / dc;
-    const int vk = 4096 / dw;  // V chunk: 16 KB (+ padding), two buffers
-    const size_t lds2 = ((((size_t)R * lcap + 1023) & ~(size_t)1023) + 2 * (size_t)(vk + 4) * dw) * 4;
-    const dim3 g2(n_kv, (M + qt2 - 1) / qt2, dc);
-    // 1024 threads for launches of few workgroups (decode: the softmax phases
-    // go 4x wider), 256 when many workgroups already fill the chip (prefill)
-    const bool wide = (size_t)g2.x * g2.y * g2.z < 1024;
-    const dim3 b2(wide ? 1024 : 256);
+    // softmax + P.V in LDS
+    if (!pv.fits) return -1;
+    const int lcap = (lmax + 7) & ~7, qt2 = pv.qt, dw = pv.dw, vk = pv.vk;
+    const size_t lds2 = pv.lds;
+    const dim3 g2(n_kv, (M + qt2 - 1) / qt2, pv.dc);
+    const bool wide = pv.threads == 1024;
+    const dim3 b2(pv.threads);
     if (hd == 64) {
         hipLaunchKernelGGL(k_attn_sc<64>, g1, dim3(256), lds1, ST(s), q, kc, pos0p, M, n_q, n_kv, max_seq, scale,
                            qt1, scores);
@@ -967,12 +1008,14 @@ void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8
     const int G = n_q / n_kv;
     if (lmax > max_seq) lmax = max_seq;
     if (prepped) *prepped = 0;
-    if (M > 1) {
+    const PvSplit pv = pv_split(M, lmax, n_kv, G, hd, true);
+    if (M > 1 && !split_first(pv, M, lmax, n_kv, G, hd, true)) {
         DpufPrep fop = op;
         if (!prepped) fop.q = NULL;
         if (attn_tile(s, M, lmax, q, NULL, NULL, &c8, out, scores, pos0, n_q, n_kv, hd, max_seq, scale, o_sign, fop) ==
             0) {
             if (fop.q) *prepped = 1;
+            attn_path_note(0);
             attn_path_note(5);
             return;
         }
@@ -988,37 +1031,22 @@ void dpuf_hip_attn_q8(void* s, int32_t M, int32_t lmax, const float* q, DpufKvQ8
         return;
     }
     // softmax + P.V: the split kernel (as the fp32 cache's) when its tile of
-    // probability rows fits in LDS, each dim chunk inside one 32-column block
-    const int lcap = (lmax + 7) & ~7;
-    const size_t budget = 112 * 1024;
-    int qt2 = 8 / G > 1 ? 8 / G : 1;
-    if (qt2 > M) qt2 = M;
-    while (qt2 > 1 && (size_t)qt2 * G * lcap * 4 > budget) qt2--;
-    if (G <= 32 && (size_t)qt2 * G * lcap * 4 <= budget) {
-        const int R = qt2 * G;
-        int dc = 1;
-        while (dc < hd / 4 && R * (hd / dc) > 256) dc *= 2;
-        const int tiles = n_kv * ((M + qt2 - 1) / qt2);
-        while (dc < hd / 4 && tiles * dc < 128) dc *= 2;
-        while (hd / dc > 32) dc *= 2;
-        const int dw = hd / dc, vk = 4096 / dw;
-        const size_t lds2 = ((((size_t)R * lcap + 1023) & ~(size_t)1023) + 2 * (size_t)(vk + 4) * dw +
-                             2 * (size_t)vk + (size_t)R * vk) * 4;
-        const dim3 g2(n_kv, (M + qt2 - 1) / qt2, dc);
-        const bool wide = (size_t)g2.x * g2.y * g2.z < 1024;
+    // probability rows fits in LDS
+    if (pv.fits) {
+        const int lcap = (lmax + 7) & ~7, qt2 = pv.qt, dw = pv.dw, vk = pv.vk;
+        const size_t lds2 = pv.lds;
+        const dim3 g2(n_kv, (M + qt2 - 1) / qt2, pv.dc);
+        const bool wide = pv.threads == 1024;
 #define PVQ(HDV, NT)                                                                                              \
     hipLaunchKernelGGL((k_attn_pv<HDV, NT, true>), g2, dim3(NT), lds2, ST(s), scores, nullptr, pos0, M, n_q, n_kv, \
                        max_seq, qt2, dw, lcap, vk, out, c8.vq, c8.vs)
-        const size_t own = (size_t)((wide ? 1024 : 256) + 2 * 32) * 4;  // the kernel's own arrays
-        if (lds2 + own <= 160 * 1024) {
-            if (hd == 64) { if (wide) PVQ(64, 1024); else PVQ(64, 256); }
-            else if (hd == 128) { if (wide) PVQ(128, 1024); else PVQ(128, 256); }
-            else { if (wide) PVQ(256, 1024); else PVQ(256, 256); }
-            LAUNCHED("k_attn_q8_sc/k_attn_pv<q8>");
-            attn_path_note(5);
-            return;
-        }
+        if (hd == 64) { if (wide) PVQ(64, 1024); else PVQ(64, 256); }
+        else if (hd == 128) { if (wide) PVQ(128, 1024); else PVQ(128, 256); }
+        else { if (wide) PVQ(256, 1024); else PVQ(256, 256); }
 #undef PVQ
+        LAUNCHED("k_attn_q8_sc/k_attn_pv<q8>");
+        attn_path_note(5);
+        return;
     }
     // rows too long for LDS: softmax in memory, P.V per (token, kv head, pair)
     const size_t lds2 = 2 * 32768 + (size_t)2 * 2 * (hd / 32) * (32768 / hd) * 4;

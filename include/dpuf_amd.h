@@ -69,15 +69,14 @@ DPUF_EXPORT uint64_t dpuf_amd_engine_weight_bytes(void* handle);
 DPUF_EXPORT int64_t dpuf_amd_engine_early_exit_count(void* handle);
 
 /* Attention launches enqueued so far in this process, by path (which: 0 the
- * matrix-instruction kernels of several tokens over the fp32 cache, 1 the
- * one-token long-context kernels (scores, softmax once per row, wide P.V; one
- * per session where they serve several), 2 the split scores + LDS softmax /
- * P.V kernels, 3 the one-pair-per-workgroup fallback, 4 the fused
- * short-context decode kernel, 5 the int8-cache kernels; and among 0 and 5:
- * 6 matrix-instruction launches whose rows are streamed, 7 the int8 cache's
- * softmax in memory); -1 for another `which`.  Enqueued, not executed: a replayed graph
- * counts at its capture only.  For tests that check which path a shape
- * takes. */
+ * matrix-instruction kernels of several tokens, 1 the one-token long-context
+ * kernels (scores, softmax once per row, wide P.V; one per session where they
+ * serve several), 2 the split scores + LDS softmax / P.V kernels over the fp32
+ * cache, 3 the one-pair-per-workgroup fallback, 4 the fused short-context
+ * decode kernel, 5 every kernel over the int8 cache; 6 those of 0 whose rows
+ * are streamed, 7 those of 5 with the softmax in memory); -1 for another
+ * `which`.  Enqueued, not executed: a replayed graph counts at its capture
+ * only.  For tests that check which path a shape takes. */
 DPUF_EXPORT int64_t dpuf_amd_attn_path_count(int32_t which);
 
 /* Times `iters` back-to-back launches of one GEMV kind over resident weights

@@ -1,8 +1,10 @@
-"""The matrix-instruction attention of several tokens (attn_tile.hip: scores,
-softmax, P.V and the O-input prep) against the oracle, bit for bit: every head
-dim and both caches, even groups that do and do not fill a 16-row tile, rows
-resident in LDS and streamed, tiles whose last rows or keys are missing, and
-scores rows that end inside a 16-byte piece."""
+"""The attention of several tokens, the matrix-instruction kernels
+(attn_tile.hip: scores, softmax, P.V and the O-input prep) and the split ones
+that take few tokens over many keys, against the oracle, bit for bit: every
+head dim and both caches, even groups that do and do not fill a 16-row tile,
+rows resident in LDS and streamed, tiles whose last rows or keys are missing,
+scores rows that end inside a 16-byte piece, and both sides of the rule that
+chooses the kernels."""
 import ctypes as C
 
 import numpy as np
@@ -15,33 +17,47 @@ from test_gpu_q8kv import Q8Pair
 
 pytestmark = pytest.mark.gpu
 
-# (query heads, KV heads, head dim, cached positions, tokens, max_seq)
+# (query heads, KV heads, head dim, cached positions, tokens, max_seq), and the
+# routes over the fp32 and the int8 cache: R / S the matrix-instruction
+# kernels with resident / streamed rows, P the split kernels (few tokens over
+# many keys: one workgroup per CU at most of 256), M the softmax in memory
 CASES = [
-    (4, 2, 64, 0, 2, 40),        # the smallest prompt
-    (4, 2, 64, 3, 37, 40),       # ends at max_seq
-    (8, 2, 128, 0, 33, 67),      # one row past a query tile; max_seq odd
-    (8, 2, 128, 61, 6, 67),      # across the first chunk boundary, up to an odd max_seq
-    (4, 2, 64, 795, 5, 810),     # resident rows, the longest (25 chunks of 32 keys)
-    (4, 2, 64, 796, 5, 810),     # streamed rows, the shortest (26 chunks)
-    (8, 2, 128, 951, 9, 970),    # resident, the longest (15 chunks of 64)
-    (8, 2, 128, 952, 9, 970),    # streamed, the shortest (16 chunks)
-    (8, 2, 128, 2042, 19, 2063), # streamed, 2061 keys
-    (12, 2, 64, 70, 23, 96),     # groups of 6: 12 of 16 rows, 30 of 32
-    (20, 2, 64, 30, 3, 64),      # groups of 10: one token per tile
-    (32, 2, 128, 17, 3, 64),     # groups of 16
-    (4, 2, 256, 120, 21, 150),   # chunks of 128 keys
-    (4, 2, 256, 480, 40, 521),   # five of them
-    (4, 2, 256, 1019, 5, 1031),  # resident, the longest (8 chunks)
-    (4, 2, 256, 1020, 5, 1031),  # streamed, the shortest (9 chunks)
-    (8, 2, 128, 7200, 2, 7240),  # half a tile of rows over many keys
+    (4, 2, 64, 0, 2, 40, "RR"),         # the smallest prompt
+    (4, 2, 64, 3, 37, 40, "RR"),        # ends at max_seq
+    (8, 2, 128, 0, 33, 67, "RR"),       # one row past a query tile; max_seq odd
+    (8, 2, 128, 61, 6, 67, "RR"),       # across the first chunk boundary, up to an odd max_seq
+    (8, 2, 128, 282, 6, 470, "RR"),     # the split kernels' range: int8 from 289 keys on
+    (8, 2, 128, 283, 6, 470, "RP"),
+    (8, 2, 128, 450, 6, 470, "RP"),     # fp32 from 457
+    (8, 2, 128, 451, 6, 470, "PP"),
+    (32, 8, 128, 600, 16, 620, "PP"),   # 256 split workgroups
+    (32, 8, 128, 600, 17, 620, "RR"),   # 288
+    (16, 8, 64, 735, 65, 810, "RR"),    # resident, the longest (25 chunks of 32 keys)
+    (16, 8, 64, 736, 65, 810, "SS"),    # streamed, the shortest
+    (32, 8, 128, 935, 25, 970, "RR"),   # resident, the longest (15 chunks of 64)
+    (32, 8, 128, 936, 25, 970, "SS"),   # streamed, the shortest
+    (32, 8, 128, 2038, 25, 2063, "SS"), # up to an odd max_seq
+    (8, 2, 128, 955, 9, 970, "PP"),
+    (8, 2, 128, 958, 9, 970, "PP"),
+    (8, 2, 128, 2042, 19, 2063, "PP"),
+    (12, 2, 64, 70, 23, 96, "RR"),      # groups of 6: 12 of 16 rows, 30 of 32
+    (20, 2, 64, 30, 3, 64, "RR"),       # groups of 10: one token per tile
+    (32, 2, 128, 17, 3, 64, "RR"),      # groups of 16
+    (32, 2, 64, 1500, 4, 1510, "PM"),
+    (4, 2, 256, 120, 21, 150, "RR"),    # chunks of 128 keys
+    (4, 2, 256, 480, 40, 521, "RP"),    # five of them
+    (16, 8, 256, 1007, 17, 1031, "RR"), # resident, the longest (8 chunks)
+    (16, 8, 256, 1008, 17, 1031, "SS"), # streamed, the shortest
+    (8, 2, 128, 7200, 2, 7240, "SS"),   # half a tile of rows, too long for the split kernels
 ]
-LONGEST_RESIDENT = {64: 800, 128: 960, 256: 1024}  # keys, by head dim
-STREAMED = 6                                       # dpuf_amd_attn_path_count: launches over streamed rows
+# dpuf_amd_attn_path_count: the tile kernels, the split ones over the fp32
+# cache, every int8 one, streamed rows, the softmax in memory
+TILES, SPLIT, INT8, STREAMED, MEMORY = 0, 2, 5, 6, 7
 
 
 @pytest.mark.parametrize("kv_type", [0, 1])
-@pytest.mark.parametrize("nq,nkv,hd,ctx,n,max_seq", CASES)
-def test_attention_of_several_tokens(eng, orc, nq, nkv, hd, ctx, n, max_seq, kv_type):
+@pytest.mark.parametrize("nq,nkv,hd,ctx,n,max_seq,routes", CASES)
+def test_attention_of_several_tokens(eng, orc, nq, nkv, hd, ctx, n, max_seq, routes, kv_type):
     shape = dict(hidden_size=256, intermediate_size=256, num_layers=2, num_q_heads=nq, num_kv_heads=nkv, head_dim=hd,
                  vocab_size=512, tie_word_embeddings=1)
     m = M.Model.build(shape, max_seq_len=max_seq, seed=401)
@@ -55,11 +71,12 @@ def test_attention_of_several_tokens(eng, orc, nq, nkv, hd, ctx, n, max_seq, kv_
             for kvh in range(nkv):
                 p.set_kv(layer, kvh, 0, rng.standard_normal((ctx, hd), dtype=np.float32),
                          rng.standard_normal((ctx, hd), dtype=np.float32))
-    path = 5 if kv_type else 0
-    c0, s0 = eng.dpuf_amd_attn_path_count(path), eng.dpuf_amd_attn_path_count(STREAMED)
+    paths = (TILES, SPLIT, INT8, STREAMED, MEMORY)
+    c0 = [eng.dpuf_amd_attn_path_count(w) for w in paths]
     lg, lo = p.forward(rng.integers(0, 512, n).astype(np.int32), ctx, only_last=0)
-    assert eng.dpuf_amd_attn_path_count(path) - c0 == 2
-    assert eng.dpuf_amd_attn_path_count(STREAMED) - s0 == (2 if ctx + n > LONGEST_RESIDENT[hd] else 0)
+    r = routes[kv_type]
+    want = (r in "RS", r == "P" and not kv_type, kv_type, r == "S", r == "M")
+    assert [eng.dpuf_amd_attn_path_count(w) - c for w, c in zip(paths, c0)] == [2 * int(w) for w in want]
     assert bits_equal(lg, lo), maxdiff(lg, lo)
     p.close()
 
@@ -86,9 +103,10 @@ def _extreme(rng, kind, keys, hd):
 
 # (the quantising store leaves finite scales of finite keys: no infinite int8 cache)
 @pytest.mark.parametrize("kind,kv_type", [("tiny", 0), ("huge", 0), ("infinite", 0), ("tiny", 1), ("huge", 1)])
-@pytest.mark.parametrize("nq,nkv,hd,ctx,n,max_seq", [
-    (4, 2, 64, 80, 9, 96), (8, 2, 128, 200, 7, 210), (8, 2, 128, 1300, 7, 1310), (8, 2, 256, 300, 5, 310)])
-def test_attention_out_of_range_values(eng, orc, nq, nkv, hd, ctx, n, max_seq, kind, kv_type):
+@pytest.mark.parametrize("nq,nkv,hd,ctx,n,max_seq,tiles", [
+    (4, 2, 64, 80, 9, 96, 1), (8, 2, 128, 200, 7, 210, 1), (32, 8, 128, 1000, 25, 1030, 1), (8, 2, 256, 270, 5, 280, 1),
+    (8, 2, 128, 1300, 7, 1310, 0)])
+def test_attention_out_of_range_values(eng, orc, nq, nkv, hd, ctx, n, max_seq, tiles, kind, kv_type):
     """Keys and values that are denormal, that overflow the scores' and the
     outputs' chains, or that are infinite or NaN (the int8 cache: its scales):
     the fp32 matrix instructions' chains round, underflow and propagate them
@@ -129,15 +147,14 @@ def test_attention_out_of_range_values(eng, orc, nq, nkv, hd, ctx, n, max_seq, k
     dq, dout, dsc, dpos = dev(q), dev(out), dev(scores), dev(np.array([ctx], np.int32))
     dkv = [dev(a) for a in host]
     scale = float(np.float32(1.0 / np.sqrt(hd)))
-    path = 5 if kv_type else 0
-    c0 = eng.dpuf_amd_attn_path_count(path)
+    c0 = eng.dpuf_amd_attn_path_count(TILES)
     if kv_type:
         L.dpuf_hip_attn_q8(None, n, keys, dq, _KvQ8(*dkv), dout, dsc, dpos, nq, nkv, hd, max_seq, scale, None, None,
                            _Prep(), None)
     else:
         assert L.dpuf_hip_attn_split(None, n, keys, dq, dkv[0], dkv[1], dout, dsc, dpos, nq, nkv, hd, max_seq, scale,
                                      None, _Prep(), None) == 0
-    assert eng.dpuf_amd_attn_path_count(path) - c0 == 1
+    assert eng.dpuf_amd_attn_path_count(TILES) - c0 == tiles
     L.dpuf_hip_d2h(M.ptr(out), dout, out.nbytes, None)
     assert L.dpuf_hip_sync(None) == 0
     for b in bufs:
