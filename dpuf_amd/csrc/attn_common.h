@@ -142,11 +142,6 @@ DEV float score_dot2(const float* q, const float* kp, int hd) {
 // keys per workgroup of the scores kernels
 #define AS_KC 64  // keys per scores workgroup
 
-// ROPE: q, k and v are the projections' raw rows; the workgroup applies the
-// QK-norm and RoPE to its group's q rows itself (as k_qk_rope_kv_w does, by
-// qk_head_rope), and the workgroup whose chunk holds the token's position
-// does the same to its K row, stores K and V to the cache at that position
-// and uses the new K row in its scores (so no launch before this one).
 // One token of each of several sessions (blockIdx.z): session z's cache bases
 // are kcs[z] + lo and vcs[z] + lo, its position pos0p[z], its q, K, V and
 // output rows q_ld / kv_ld apart, and its score rows sc_ld.
@@ -158,6 +153,11 @@ struct MsTab {
     size_t sc_ld;
 };
 
+// ROPE: q, k and v are the projections' raw rows; the workgroup applies the
+// QK-norm and RoPE to its group's q rows itself (as k_qk_rope_kv_w does, by
+// qk_head_rope), and the workgroup whose chunk holds the token's position
+// does the same to its K row, stores K and V to the cache at that position
+// and uses the new K row in its scores (so no launch before this one).
 struct ScRope {
     const float* k;  // raw K and V of the token [n_kv][HD]
     const float* v;
@@ -278,10 +278,6 @@ DEV float pv_chain(const float* p, const float* v, int n, float a) {
 // and the wide P.V; -1 (nothing launched) when the shape does not take them.
 // wm (or NULL): the weight groups that warm-up workgroups of the P.V launch
 // read into the caches on the CUs its chain workgroups leave idle.
-int32_t attn_wide_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v, const float* qn,
-                           const float* kn, float eps, const float* cos_tab, const float* sin_tab, float* const* kcs,
-                           float* const* vcs, size_t lo, float* out, float* scores, const int32_t* pos, int32_t n_q,
-                           int32_t n_kv, int32_t hd, int32_t max_seq, float scale);
 int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, const float* vc, float* out,
                       float* scores, const int32_t* pos0p, int32_t n_q, int32_t n_kv, int32_t hd, int32_t max_seq,
                       float scale, const ScRope* rope, const DpufWarm* wm);
@@ -290,6 +286,14 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
 // weights that warm-up workgroups of the P.V launch read into the caches.
 int32_t attn_wide_q8(void* s, int32_t lmax, const int32_t* pos0, int32_t n_q, int32_t n_kv, int32_t hd,
                      int32_t max_seq, float* scores, float* out, DpufKvQ8 c8, const DpufWarm* wm);
+
+// One token of each of n sessions over the fp32 cache, the longest having lmax
+// keys, through the same kernels with a session axis; -1 (nothing launched)
+// when the shape does not take them.
+int32_t attn_wide_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v, const float* qn,
+                           const float* kn, float eps, const float* cos_tab, const float* sin_tab, float* const* kcs,
+                           float* const* vcs, size_t lo, float* out, float* scores, const int32_t* pos, int32_t n_q,
+                           int32_t n_kv, int32_t hd, int32_t max_seq, float scale);
 
 // The attention of M > 1 tokens on the fp32 matrix instructions
 // (attn_tile.hip), even groups of up to 16 heads, over the fp32 cache (kc, vc)

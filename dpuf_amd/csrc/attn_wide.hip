@@ -888,9 +888,10 @@ int32_t attn_wide_f32(void* s, int32_t lmax, const float* q, const float* kc, co
 // slot's cache (tables kcs / vcs, positions pos), in the three launches of the
 // longest session alone: QK-norm, RoPE, KV store and scores; softmax; P.V.
 // One by one, five sessions of 200 to 2 600 keys took 15 launches and 85 us per
-// layer at the 8B width; together 33.  Every session takes the kernels it would take
-// alone, so its results are the same bits.  Groups of 2 and 4; -1 with nothing
-// launched otherwise.
+// layer at the 8B width; together 33.  The kernels keep the reference's order
+// whatever the length, so a session's results are the same bits as alone, also
+// for one of up to 192 keys, which alone takes the fused decode kernel.  Groups
+// of 2 and 4; -1 with nothing launched otherwise.
 int32_t attn_wide_sessions(void* s, int32_t n, int32_t lmax, float* q, const float* k, const float* v, const float* qn,
                            const float* kn, float eps, const float* cos_tab, const float* sin_tab, float* const* kcs,
                            float* const* vcs, size_t lo, float* out, float* scores, const int32_t* pos, int32_t n_q,

@@ -76,10 +76,9 @@ typedef struct {
     void* d_lmred;
     /* one token per session (dpuf_amd_engine_forward_slots): while ms_n > 0
      * the layers run ms_n tokens, token m of slot ms_slot[m] at position
-     * ms_pos[m] (device copy d_ms_pos); the first ms_short of them (fp32
-     * cache, at most DPUF_HIP_DEC_MAX_KEYS keys) through one fused decode
-     * attention launch with the KV caches at d_ms_kc[m] / d_ms_vc[m], every
-     * other one through the one-token attention launches of its own slot */
+     * ms_pos[m] (device copy d_ms_pos) against the KV caches at d_ms_kc[m] /
+     * d_ms_vc[m] (fp32 cache).  The first ms_short of them have at most
+     * DPUF_HIP_DEC_MAX_KEYS keys; enqueue_ms_attention has the launches */
     int32_t ms_n, ms_short;
     int32_t ms_slot[DPUF_AMD_MAX_BATCH], ms_pos[DPUF_AMD_MAX_BATCH];
     int32_t *d_ms_pos, *d_ms_tok;

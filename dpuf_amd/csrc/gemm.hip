@@ -67,8 +67,8 @@
 //
 // us per launch at the 8B widths, before (one 16-row x 64-token fp16 tile per
 // wave for every M) -> now: down M = 29 85 -> 27, M = 90 93 -> 37, M = 512 144
-// -> 108; O 30 -> 11, 31 -> 15, 47.5 -> 39; mode 14 down M = 90 135 -> 48, M =
-// 512 223 -> 145; gate + up M = 512 225 -> 181.
+// -> 108; O 30 -> 11, 31 -> 15, 47.5 -> 38; mode 14 down M = 90 135 -> 50, M =
+// 512 223 -> 145; gate + up with the SwiGLU M = 512 202 -> 178.
 // ---------------------------------------------------------------------------
 
 #define GM_SWI_ROWS 16384  // gate + up rows from which the fused SwiGLU launch pays
