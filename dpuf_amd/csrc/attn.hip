@@ -870,13 +870,14 @@ static PvSplit pv_split(int M, int lmax, int n_kv, int G, int hd, bool q8) {
 // dim; a few tokens over many keys are a few such workgroups, while the split
 // P.V gives each a fraction of the dims.  So the split kernels win as long as
 // their grid is one workgroup per CU at most, from a length on that grows with
-// what a workgroup repeats or shares.  us per layer, split | tiles, 8 KV heads,
-// groups of 4, head dim 128, fp32: 2 tokens at 300 keys 57 | 55, 600 61 | 62,
-// 1 100 64 | 79, 2 000 74 | 106, 4 000 87 | 162; 16 tokens (256 workgroups) at
-// 4 000 139 | 171, 24 (384) 214 | 178.  int8 cache: 2 tokens at 4 000 98 | 169,
-// 24 at 4 000 287 | 189.  The int8 softmax in memory, where the split kernel's
-// rows do not fit LDS, wins likewise at head dim 64 only (groups of 16, 2
-// tokens at 4 000 163 | 196; head dim 128, groups of 8, 187 | 173).
+// what a workgroup repeats or shares.  us per layer of a model of width 256 (about
+// 45 of them not attention), split | tiles, 8 KV heads, groups of 4, head dim 128,
+// fp32: 2 tokens at 300 keys 56 | 54, 600 59 | 61, 1 100 64 | 78, 2 000 71 | 102,
+// 4 000 88 | 162; 16 tokens (256 workgroups) at 4 000 138 | 171, 24 (384) 213 |
+// 178.  int8 cache: 2 tokens at 4 000 99 | 169, 24 at 4 000 287 | 189.  The int8
+// softmax in memory, where the split kernel's rows do not fit LDS, wins likewise
+// at head dim 64 only (groups of 16, 2 tokens at 4 000 163 | 196; head dim 128,
+// groups of 8, 190 | 173).
 static bool split_first(const PvSplit& p, int M, int lmax, int n_kv, int G, int hd, bool q8) {
     const int n_cu = dpuf_hip_cu_count();
     if (lmax <= (q8 ? 48 * G + 96 : 3 * hd + 8 * G + 40)) return false;
